@@ -471,13 +471,16 @@ void prefill_fwd(const PrefillArgs a) {
   const int qi = q0 + rg * 32 + l32;                     // this lane's query row
 
   // ---- Q^T operand (B of S^T = K Q^T): query qi, d = 16 j + 8 h + [0, 8)
-  // (loaded by load_q below, after the first K block's transfers are issued)
+  // (through LDS, see dma_q, or straight into registers)
+  constexpr bool kQLds = S == 4 ? ROPE == kRopeNone : D >= 128;
   u32x4 qop[KST];
-  RopeQ<D, ROPE> rq;   // rotation inputs (applied once the first K/V transfers are issued)
   auto load_q = [&]() {
     const char* qp = a.q + b * a.q_sb + (int64_t)hq * a.q_sh + (int64_t)min(qi, a.Tq - 1) * a.q_sm + 16 * h;
 #pragma unroll
     for (int j = 0; j < KST; ++j) qop[j] = *(const u32x4*)(qp + 32 * j);   // (rows past Tq read row Tq - 1; never stored)
+  };
+  RopeQ<D, ROPE> rq;   // rotation inputs (applied once the first K/V transfers are issued)
+  auto load_tables = [&]() {
     if constexpr (ROPE != kRopeNone) {
       const int64_t base = (int64_t)a.start_host + (a.start_pos != nullptr ? a.start_pos[a.pos_per_seq ? b : 0] : 0);
       rope_q_fetch<D, ROPE>(a, rq, base + qi, h);
@@ -579,6 +582,32 @@ void prefill_fwd(const PrefillArgs a) {
   // buffer range: the hardware drops every out-of-range read (no memory
   // traffic) and what it fills is never read, so every wave issues the same
   // instruction count per group and the waits below are constants.
+  // kQLds: q comes through LDS, a wave's 32 rows by 1 KB LDS DMA (whole rows,
+  // swizzled like the K stages) into a part of the ring that the first blocks
+  // do not use yet, then read in the operand layout.  Loaded straight into
+  // registers, each of a wave's q instructions touches 32 rows (256 cache-line
+  // requests per wave at D = 128 instead of 64).  Per call, straight -> LDS:
+  // head_dim 256 one sequence of 500 tokens 27.4 -> 26.4 us, 1000 tokens with
+  // the rotary prologue 62.2 -> 56.2, head_dim 128 512 tokens 15.2 -> 14.9.
+  // Rows of 128 bytes and less gain nothing (D = 32, 2 x 700 tokens: 12.3 ->
+  // 12.6), nor does the rotary prologue of the four-stage ring (B4 x 2048:
+  // 161.7 -> 163.7), whose table loads set its time.  Rows past Tq read row
+  // Tq - 1; they are never stored.
+  auto dma_q = [&](char* qst) {
+    const char* qb = a.q + b * a.q_sb + (int64_t)hq * a.q_sh;
+#pragma unroll
+    for (int i = 0; i < 32 * RB / 1024; ++i) {
+      const int r = i * ROWS_PER_DMA + lane / NC;
+      const char* src = qb + (int64_t)min(q0 + rg * 32 + r, a.Tq - 1) * a.q_sm + (((lane % NC) ^ (r % NC)) * 16);
+      char* dst = qst + i * 1024;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+  };
+  auto read_q = [&](const char* qst) {
+#pragma unroll
+    for (int j = 0; j < KST; ++j) qop[j] = *(const u32x4*)(qst + k_rd[j]);
+  };
   // (one transfer instruction each: the ring refills are spread over the
   // MFMA stream, see `qk`)
   auto issue_k1 = [&](int blk, char* LK, int i) {
@@ -973,62 +1002,37 @@ void prefill_fwd(const PrefillArgs a) {
         for (int p = 0; p < NP; ++p) piece1(p);
       }
     };
-    // Prologue: K_0's transfers first, then q (its 32 rows per load
-    // instruction take the memory pipeline a while), then V_0, K_1, K_2,
-    // V_1.  The first scores wait for K_0 and q only; the rest land under
-    // them.  (Loads retire in order, so vmcnt(later) covers exactly K_0 and
-    // q.)
-    if (nblk > 0) {
-      if constexpr (ROPE == kRopeNone) {
-        // q comes through LDS: each wave's 32 rows by 1 KB LDS DMA (whole
-        // rows, swizzled like the K stages) into a stage the first blocks do
-        // not use yet (V_1's, K_3's, V_2's, V_3's; 2 waves each), then read in
-        // the operand layout.  Loaded straight into registers, each of a
-        // wave's q instructions touched 32 rows (256 cache-line requests per
-        // wave instead of 64), and the memory pipeline worked through them
-        // ahead of the ring's first transfers.  Rows past Tq read as zeros.
-        issue_k(0, lk0);
-        issue_v(0, lv0);
-        issue_k(1, lk1);
-        issue_k(2, lk2);
-        char* qst = ((wave >> 1) == 0 ? lv1 : (wave >> 1) == 1 ? lk3 : (wave >> 1) == 2 ? lv2 : lv3) +
-                    (wave & 1) * 32 * RB;
-        {
-          const int r0w = q0 + rg * 32;
-          const int nrow = max(0, min(32, a.Tq - r0w));
-          const int bytes = nrow > 0 ? (nrow - 1) * (int)a.q_sm + RB : 0;
-          const __amdgpu_buffer_rsrc_t rsq = __builtin_amdgcn_make_buffer_rsrc(
-              (void*)(a.q + b * a.q_sb + (int64_t)hq * a.q_sh + (int64_t)min(r0w, a.Tq - 1) * a.q_sm), 0, bytes,
-              kBufferFlags);
-#pragma unroll
-          for (int i = 0; i < 32 * RB / 1024; ++i) {
-            const int r = i * ROWS_PER_DMA + lane / NC;
-            const int voff = r * (int)a.q_sm + (((lane % NC) ^ (r % NC)) * 16);
-            char* dst = qst + i * 1024;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsq, dst, 16, voff, 0, 0, 0);
-          }
-        }
-        wait_vmcnt<0>();                                  // this wave's q (and K_0 .. K_2, V_0) landed
-#pragma unroll
-        for (int j = 0; j < KST; ++j) qop[j] = *(const u32x4*)(qst + k_rd[j]);
-        ring_barrier();                                   // every wave's q read and K_0 landed
-        issue_v(1, lv1);                                  // into the q stage just read
-        first_scores();
-      } else {
-        issue_k(0, lk0);
-        load_q();
-        __builtin_amdgcn_sched_barrier(0);
-        issue_v(0, lv0);
-        issue_k(1, lk1);
-        issue_k(2, lk2);
-        issue_v(1, lv1);
-        wait_vmcnt<2 * NK + 2 * NV>();
-        rope_q_apply<D, T, ROPE>(a, qop, rq, h);
-        ring_barrier();
-        first_scores();
-      }
-    } else {
+    // Prologue through LDS: K_0, V_0, K_1, K_2 and q, whose stages (V_1's,
+    // K_3's, V_2's, V_3's; 2 waves each) the first blocks do not use yet; V_1
+    // follows once every wave has read its q.  Straight: K_0, q and the
+    // tables, then V_0, K_1, K_2, V_1, which land under the first scores
+    // (loads retire in order, so the wait covers exactly K_0, q and tables).
+    if (nblk > 0 && !kQLds) {
+      issue_k(0, lk0);
       load_q();
+      load_tables();
+      __builtin_amdgcn_sched_barrier(0);
+      issue_v(0, lv0);
+      issue_k(1, lk1);
+      issue_k(2, lk2);
+      issue_v(1, lv1);
+      wait_vmcnt<2 * NK + 2 * NV>();
+      if constexpr (ROPE != kRopeNone) rope_q_apply<D, T, ROPE>(a, qop, rq, h);
+      ring_barrier();
+      first_scores();
+    } else if (nblk > 0) {
+      issue_k(0, lk0);
+      char* qst = ((wave >> 1) == 0 ? lv1 : (wave >> 1) == 1 ? lk3 : (wave >> 1) == 2 ? lv2 : lv3) +
+                  (wave & 1) * 32 * RB;
+      issue_v(0, lv0);
+      issue_k(1, lk1);
+      issue_k(2, lk2);
+      dma_q(qst);
+      wait_vmcnt<0>();                                    // this wave's q (and K_0 .. K_2, V_0) landed
+      read_q(qst);
+      ring_barrier();                                     // every wave's q read and K_0 landed
+      issue_v(1, lv1);                                    // into the q stage just read
+      first_scores();
     }
     // blocks 0 .. nblk - 2 in full steps, then the last block's PV product
     int j = 0;
@@ -1057,11 +1061,14 @@ void prefill_fwd(const PrefillArgs a) {
       pack_vstage(vstage(PfParity<P>{}));                // variant 2: V_j's image (its rows have landed)
       work(parity, j, sa0, sa1, sb0, sb1, rmax, no_piece);
     };
-    // Prologue as on the four-stage ring: K_0, q, then V_0 and K_1 landing
-    // under the first scores.
-    if (nblk > 0) {
+    // Prologue through LDS: the tables (the wait for q covers them), K_0, q
+    // into the V stages, K_1; V_0 follows once every wave has read its q and
+    // lands with K_1 under the first scores.  Straight: as on the four-stage
+    // ring.
+    if (nblk > 0 && !kQLds) {
       issue_k(0, lk0);
       load_q();
+      load_tables();
       __builtin_amdgcn_sched_barrier(0);
       issue_v(0, lv0);
       issue_k(1, lk1);
@@ -1069,8 +1076,19 @@ void prefill_fwd(const PrefillArgs a) {
       if constexpr (ROPE != kRopeNone) rope_q_apply<D, T, ROPE>(a, qop, rq, h);
       ring_barrier();
       first_scores();
-    } else {
-      load_q();
+    } else if (nblk > 0) {
+      load_tables();
+      __builtin_amdgcn_sched_barrier(0);
+      issue_k(0, lk0);
+      char* qst = ((wave >> 1) == 0 ? lv0 : lv1) + (wave & 1) * 32 * RB;
+      dma_q(qst);
+      issue_k(1, lk1);
+      wait_vmcnt<NK>();                                   // this wave's K_0 and q landed
+      read_q(qst);
+      if constexpr (ROPE != kRopeNone) rope_q_apply<D, T, ROPE>(a, qop, rq, h);
+      ring_barrier();
+      issue_v(0, lv0);
+      first_scores();
     }
     int j = 0;
     for (; j + 1 < nfb; j += 2) {
