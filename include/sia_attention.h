@@ -178,7 +178,9 @@ int sia_paged_gqa_int8_flash_decode_noalloc(const sia_tensor* q, const sia_tenso
  * workspace: device memory of at least sia_prefill_workspace_size bytes
  * (256-byte aligned); it holds V converted to f16 in the kernel's block
  * layout (float16 V at head_dim 32-128 needs none: NULL, 0 is accepted
- * there) and is free again when the stream passes the call.  f32 inputs run in fp32 on the vector
+ * there) and is free again when the stream passes the call.  With
+ * sia_attention_flash_fwd_workspace_size bytes a call of few query rows over
+ * many keys may also split its keys.  f32 inputs run in fp32 on the vector
  * ALUs and need no workspace (NULL, 0 is accepted). */
 int sia_attention_flash_fwd(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int32_t causal,
                             float sm_scale, const sia_tensor* out, void* workspace, size_t workspace_bytes,
@@ -210,6 +212,13 @@ int sia_attention_flash_fwd_rope(const sia_tensor* q, const sia_tensor* k, const
  * (batch, kv_heads, kv_len, head_dim).  No reference counterpart: the
  * reference's Triton launch allocates nothing (kernels/attention_kernel.py:296). */
 int sia_prefill_workspace_size(int64_t batch, int64_t kv_heads, int64_t kv_len, int64_t head_dim, size_t* bytes);
+
+/* Workspace bytes with which the call of these q and k (shapes and dtypes
+ * only) may also split its keys over work-groups: at least what
+ * sia_prefill_workspace_size asks for, plus fp32 partials when few query rows
+ * face many keys (a short prompt over a long cached prefix).  With a smaller
+ * workspace such a call runs unsplit. */
+int sia_attention_flash_fwd_workspace_size(const sia_tensor* q, const sia_tensor* k, size_t* bytes);
 
 /* ------------------------------------------------------------ KV write path */
 

@@ -33,6 +33,72 @@ int64_t image_bytes(int64_t B, int64_t Hkv, int64_t Tk, int64_t D) {
   return B * Hkv * nkb * kPfBN * DV * 2;
 }
 
+// Work-groups of a launch with `var`'s geometry.
+int64_t groups(int64_t B, int64_t Hkv, int64_t G, int64_t Tq, int D, int var) {
+  const int h = pf_heads_per_group(D, (int)G, var);
+  const int64_t r = 32 * pf_waves(D, var) / h;
+  return ((Tq + r - 1) / r) * (B * Hkv * (G / h));
+}
+
+// How a call's keys are split over work-groups: `ns` runs (1: not split) on
+// prefill_fwd variant `var`, whose partials take `bytes` after the V^T images.
+struct KeySplit {
+  int ns = 1, var = 0;
+  int64_t bytes = 0;
+};
+
+// A call whose work-groups cover at most half of the CUs' slots leaves the
+// others idle while each group walks every key block (200 query rows over
+// 6200 keys: 56 groups of 97 blocks, 101 us).  Its time is estimated, split
+// and not, in microseconds: a fixed part (prologue, last block, stores and,
+// split, the merge), the chain of key blocks of one group, longer when two
+// groups share a CU, the V repack, and the fp32 partials written and read.
+// The constants are fitted to back-to-back calls at 32/8 and 16/4 heads,
+// 5-1000 rows over 1000-8192 keys (estimates within 10% there).  Split where
+// that promises a fifth: per call, unsplit -> split, bf16 head_dim 128
+// 5 + 8192 tokens 128 -> 17 us, 64 + 3000 52 -> 19, 200 + 6000 101 -> 42,
+// 512 + 8192 136 -> 84; head_dim 256 200 + 6000 176 -> 48; prompts without a
+// prefix stay whole (512 tokens 15.5 against 25 us in two runs, 1024 25
+// against 39: the partials and the merge cost more than the chain saves).
+KeySplit key_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, int64_t D, bool bf16, int cus) {
+  KeySplit best;
+  const int64_t nkb = (Tk + kPfBN - 1) / kPfBN;
+  if ((D != 64 && D != 128 && D != 256) || Tq <= 0 || nkb < 8 || cus <= 0) return best;
+  const int64_t rows = B * Hq * Tq, row_bytes = (D + 2) * 4;
+  const int64_t most_bytes = (int64_t)256 << 20;      // (also keeps rows below 2^31, as the merge indexes them)
+  const double fixed = 8.5;
+  const double blk = D == 64 ? 0.85 : D == 128 ? 0.95 : 1.73;      // one group alone on a CU
+  const double conv = bf16 ? (D == 64 ? 0.15 : 0.3) : 0.0;         // V block converted in LDS
+  const double pack = bf16 || D == 256 ? 3.0 + 4.0 * D * Tk * Hkv * B / 4.6e6 : 0.0;
+  const bool in_lds = D <= 128 && bf16 && Tk <= (D == 64 ? kPackvMaxKeysD64 : kPackvMaxKeys);   // (variant 2)
+  double limit = 0.8 * (fixed + (in_lds ? (blk + conv) * nkb : blk * nkb + pack));
+  struct Way { int var; double blk, pack, shared; int64_t slots; };
+  const Way ways[2] = {
+      // variant 3: bf16 V converted in LDS block by block (head_dim 256 and
+      // float16 at head_dim 64 run variant 4)
+      {3, blk + conv, 0.0, D == 64 ? 1.3 : 1.6, 2 * (int64_t)cus},
+      // variant 4: variant 0's groups, V^T images
+      {4, D == 128 ? 1.54 : blk, pack, D == 64 ? 1.3 : 1.0, D == 64 ? 2 * (int64_t)cus : cus}};
+  for (const Way& w : ways) {
+    const bool built = w.var == 3 ? D == 128 || (D == 64 && bf16)
+                                  : D == 256 || (D == 64 && !bf16) || (D == 128 && bf16);
+    if (!built) continue;
+    const int64_t wg = groups(B, Hkv, Hq / Hkv, Tq, (int)D, w.var);
+    const int64_t most = w.slots / wg < nkb / 2 ? w.slots / wg : nkb / 2;
+    for (int64_t n = 2; n <= most && n <= 64 && rows * n * row_bytes <= most_bytes; ++n) {
+      const int64_t bps = (nkb + n - 1) / n, ns = (nkb + bps - 1) / bps;
+      const double t = fixed + w.pack + bps * w.blk * (wg * ns > cus ? w.shared : 1.0) + rows * ns * D * 8 / 5e6;
+      if (ns > 1 && t < limit) {
+        limit = t;
+        best.ns = (int)ns;
+        best.var = w.var;
+      }
+    }
+  }
+  if (best.ns > 1) best.bytes = rows * best.ns * row_bytes;   // O rows, then (max, sum) pairs
+  return best;
+}
+
 // Float32 q/k/v: the vector-ALU path (attn_f32.hpp), one work item per
 // (sequence, KV head, chunk of query rows x heads), no workspace.
 int prefill_f32(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int32_t causal, float sm_scale,
@@ -184,12 +250,14 @@ int flash_fwd(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int
   // At D = 128, a grid of at most one 8-wave group per CU runs as 4-wave
   // groups instead (prefill_fwd variant 1): twice the groups, each with half
   // the rows.  (Up to two 8-wave groups per CU this was measured slower.)
-  auto groups = [&](int var) {
-    const int h = pf_heads_per_group((int)D, a.G, var);
-    const int64_t r = 32 * pf_waves((int)D, var) / h;
-    return ((Tq + r - 1) / r) * (B * Hkv * (a.G / h));
-  };
-  L.var = D == 128 && groups(0) <= dev.cus ? 1 : 0;
+  L.var = D == 128 && groups(B, Hkv, a.G, Tq, (int)D, 0) <= dev.cus ? 1 : 0;
+  // Few query rows over many keys: variant 3 or 4, when the caller's workspace
+  // also holds the partials (the size of sia_attention_flash_fwd_workspace_size)
+  const KeySplit ks = v_rows_ok ? key_splits(B, Hq, Hkv, Tq, Tk, D, q->dtype == SIA_BF16, dev.cus) : KeySplit();
+  const int64_t images = ks.var == 4 ? need : 0;         // (variant 3 needs none)
+  if (ks.ns > 1 && workspace != nullptr && (uintptr_t)workspace % 256 == 0 &&
+      workspace_bytes >= (size_t)(images + ks.bytes))
+    L.var = ks.var;
   const int hpw = pf_heads_per_group((int)D, a.G, L.var);
   int lg = 0;
   while ((1 << lg) < hpw) ++lg;
@@ -197,6 +265,16 @@ int flash_fwd(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int
   const int rows = 32 * pf_waves((int)D, L.var) / hpw;
   a.nqblk = (int)((Tq + rows - 1) / rows);
   a.nkb = (int)((Tk + kPfBN - 1) / kPfBN);
+  if (L.var >= 3) {
+    a.nsplit = ks.ns;
+    a.bps = (a.nkb + ks.ns - 1) / ks.ns;
+    a.nrows = B * Hq * Tq;
+    a.part_o = (float*)((char*)workspace + images);
+    a.part_ml = a.part_o + a.nrows * a.nsplit * D;
+    a.dS = make_fastdiv((uint32_t)a.nsplit);
+    a.dTq = make_fastdiv((uint32_t)Tq);
+    a.dHq = make_fastdiv((uint32_t)Hq);
+  }
   const int64_t nunit = B * Hkv * (a.G / hpw);
   if ((int64_t)a.nqblk * nunit > 0x7fffffff || B * Hkv > 0x7fffffff)
     return fail(SIA_ERR_UNSUPPORTED, "grid too large");
@@ -229,6 +307,11 @@ int flash_fwd(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int
     // them transposed from LDS (no V^T images, no repack)
     a.v = p.v; a.v_sb = p.v_sb; a.v_sh = p.v_sh; a.v_sn = v_sn;
     p.nblocks = 0;
+  } else if (L.var == 3) {
+    a.v = p.v; a.v_sb = p.v_sb; a.v_sh = p.v_sh; a.v_sn = v_sn;
+    p.nblocks = 0;
+  } else if (L.var == 4) {
+    // the V^T images of variant 0
   } else if (q->dtype == SIA_BF16 && (L.var == 1 || ((D == 32 || D == 64) && L.var == 0)) &&
              Tk <= (D <= 64 ? kPackvMaxKeysD64 : kPackvMaxKeys) &&
              (int64_t)a.nqblk * nunit <= 2 * (int64_t)dev.cus &&
@@ -256,6 +339,25 @@ extern "C" int sia_prefill_workspace_size(int64_t batch, int64_t kv_heads, int64
     return fail(SIA_ERR_UNSUPPORTED, "prefill head_dim %lld not supported (16, 32, 64, 128, 256)",
                 (long long)head_dim);
   *bytes = (size_t)image_bytes(batch, kv_heads, kv_len, head_dim);
+  return SIA_OK;
+}
+
+extern "C" int sia_attention_flash_fwd_workspace_size(const sia_tensor* q, const sia_tensor* k, size_t* bytes) {
+  if (bytes == nullptr || q == nullptr || k == nullptr) return fail(SIA_ERR_INVALID_ARGUMENT, "q, k or bytes is NULL");
+  if (q->ndim != 4 || k->ndim != 4) return fail(SIA_ERR_INVALID_ARGUMENT, "q and k must have 4 dims");
+  const int64_t B = q->shape[0], Hq = q->shape[1], Tq = q->shape[2], D = q->shape[3];
+  const int64_t Hkv = k->shape[1], Tk = k->shape[2];
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Tq < 0 || Tk < 0) return fail(SIA_ERR_INVALID_ARGUMENT, "bad sizes");
+  if (Hq % Hkv) return fail(SIA_ERR_INVALID_ARGUMENT, "Hq must be a multiple of Hkv");
+  if (!head_dim_ok(D))
+    return fail(SIA_ERR_UNSUPPORTED, "prefill head_dim %lld not supported (16, 32, 64, 128, 256)", (long long)D);
+  *bytes = 0;
+  if (q->dtype == SIA_F32) return SIA_OK;
+  const int64_t images = q->dtype == SIA_F16 && D >= 32 && D <= 128 ? 0 : image_bytes(B, Hkv, Tk, D);
+  const KeySplit ks = key_splits(B, Hq, Hkv, Tq, Tk, D, q->dtype == SIA_BF16, device_info().cus);
+  // (variant 3 reads no V^T images, but the call asks for room for them in any case)
+  const int64_t used = (ks.var == 4 ? images : 0) + ks.bytes;
+  *bytes = (size_t)(used > images ? used : images);
   return SIA_OK;
 }
 

@@ -10,8 +10,7 @@ static int launch_fwd(PrefillLaunch& L, int rope);
 
 template <int D, class T>
 static int launch_prefill_typed(PrefillLaunch& L) {
-  // rotary variant: none, or split-half / interleaved pairs from 16-bit / fp32 tables
-  const int rope = L.a.cs == nullptr ? kRopeNone : 1 + (L.a.interleaved ? 1 : 0) + (L.a.tab_dt == SIA_F32 ? 2 : 0);
+  const int rope = rope_variant(L.a);
   if (L.pack.nblocks > 0) {
     // one work-group per 64-key V^T image
     hipLaunchKernelGGL((prefill_pack_v<D, T>), dim3((unsigned)L.pack.nblocks), dim3(256), 0, L.stream, L.pack);
@@ -22,6 +21,7 @@ static int launch_prefill_typed(PrefillLaunch& L) {
     if (L.var == 2) return launch_fwd<D, T, 2>(L, rope);
   if constexpr (D == 128)
     if (L.var == 1) return launch_fwd<D, T, 1>(L, rope);
+  if (L.var >= 3) return launch_prefill_split(L);
   // (a variant the host picked but this head_dim/dtype has no kernel for
   // would run the images path on V^T images nobody wrote)
   if (L.var != 0) return fail(SIA_ERR_LAUNCH, "prefill variant %d is not built for head_dim %d", L.var, D);

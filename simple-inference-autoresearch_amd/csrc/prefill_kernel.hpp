@@ -78,6 +78,13 @@ struct PrefillArgs {
   const char* cs; const char* sn; int64_t tab_rs;
   int32_t Tc, tab_dt, interleaved;
   const int32_t* start_pos; int32_t start_host, pos_per_seq;
+  // variants 3 and 4: the key blocks are cut into nsplit runs of bps blocks, one
+  // work-group each; a run's fp32 partial of row ((b Hq + hq) Tq + i) is
+  // part_o[split][row][D] and part_ml[split][row] = (max, sum)
+  float* part_o; float* part_ml;
+  int32_t nsplit, bps;
+  int64_t nrows;                                // B * Hq * Tq
+  FastDiv dS, dTq, dHq;                         // divisions by nsplit (kernel), Tq and Hq (merge)
 };
 
 struct PackArgs {
@@ -104,6 +111,11 @@ constexpr int kBufferFlags = 0x00020000;   // gfx9 raw buffer resource word 3 (3
 //    where the call is launch- and latency-bound).
 //    float16 at D = 32 ... 128 needs no V^T images in any variant: raw V rows
 //    and transposed LDS reads (kTrV in prefill_fwd).
+//    Variants 3 (variant 2's groups; D = 64, 128) and 4 (variant 0's groups;
+//    D = 64, 128, 256) give each work-group one run of the key blocks and
+//    merge the runs' fp32 partials in prefill_merge: few query rows over many
+//    keys, where whole calls leave most CUs idle (chosen by key_splits in
+//    capi_prefill.cpp, which holds the measurements).
 //  * D <= 64: 4 waves with the same register budget, so two work-groups share
 //    a CU and one's prologue and epilogue overlap the other's key loop (MHA
 //    D = 64 at T = 1024: 88 -> 70 us per call); a two-stage ring at D = 64,
@@ -115,8 +127,9 @@ constexpr int kBufferFlags = 0x00020000;   // gfx9 raw buffer resource word 3 (3
 // dimensions wide (D = 16 is zero-padded).
 template <int D, int VAR = 0>
 struct PfCfg {
-  static constexpr bool small = VAR >= 1;
-  static constexpr bool packv = VAR == 2;                 // V^T images built in LDS from raw V rows
+  static constexpr bool small = VAR >= 1 && VAR <= 3;
+  static constexpr bool packv = VAR == 2 || VAR == 3;     // V converted in LDS from raw V rows
+  static constexpr bool split = VAR >= 3;                 // one run of key blocks per work-group, fp32 partials
   static constexpr int waves = D == 128 && !small ? 8 : 4;
   static constexpr int stages = small ? 2 : D == 128 || D < 64 ? 4 : 2;
   static constexpr int wpe = D <= 128 ? 2 : 1;          // waves per SIMD the registers are budgeted for
@@ -131,7 +144,7 @@ struct PfCfg {
 };
 
 // Waves per work-group of prefill_fwd at head_dim D (host side).
-inline int pf_waves(int D, int var = 0) { return D == 128 && var == 0 ? 8 : 4; }
+inline int pf_waves(int D, int var = 0) { return D == 128 && (var == 0 || var == 4) ? 8 : 4; }
 // Query heads per work-group: the largest power of two that divides the GQA
 // group size G and is at most the wave count (host side).
 inline int pf_heads_per_group(int D, int G, int var = 0) {
@@ -381,11 +394,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // (one template argument each: __launch_bounds__ is a macro)
-template <int C> constexpr int kPfThreads = PfCfg<C / 4, C % 4>::waves * 64;
-template <int C> constexpr int kPfWpe = PfCfg<C / 4, C % 4>::wpe;
+template <int C> constexpr int kPfThreads = PfCfg<C / 8, C % 8>::waves * 64;
+template <int C> constexpr int kPfWpe = PfCfg<C / 8, C % 8>::wpe;
 
 template <int D, class T, int ROPE, int VAR>
-__global__ __launch_bounds__(kPfThreads<4 * D + VAR>) __attribute__((amdgpu_waves_per_eu(kPfWpe<4 * D + VAR>)))
+__global__ __launch_bounds__(kPfThreads<8 * D + VAR>) __attribute__((amdgpu_waves_per_eu(kPfWpe<8 * D + VAR>)))
 void prefill_fwd(const PrefillArgs a) {
   using C = PfCfg<D, VAR>;
   constexpr int NW = C::waves, S = C::stages, DV = C::DV;
@@ -432,10 +445,10 @@ void prefill_fwd(const PrefillArgs a) {
   // work-group fold + i the second slot of work-group i's CU.  Those are
   // numbered lightest-first, so every CU pairs a heavy and a light group
   // (per XCD with the XCD-aware order, whose slots fold the same way).
-  int ql, u;
+  int ql, u, split = 0;
   {
     const int lin = blockIdx.x;
-    const int nall = a.nqblk * a.nunit;
+    const int nall = a.nqblk * a.nunit * (C::split ? a.nsplit : 1);
     const int xcd = lin & 7;
     const int slot0 = lin >> 3, f8 = a.fold >> 3;
     const int slot = a.fold && slot0 >= f8 ? f8 + ((nall >> 3) - 1 - slot0) : slot0;
@@ -446,7 +459,16 @@ void prefill_fwd(const PrefillArgs a) {
     const int u1 = lin1 - ql1 * a.nunit;
     ql = a.remap ? ql8 : ql1;
     u = a.remap ? u8 : u1;
+    if constexpr (C::split) {   // (query block, run of key blocks), runs fastest
+      const int q = fdiv(ql, a.dS);
+      split = ql - q * a.nsplit;
+      ql = q;
+    }
   }
+  // variants 3 and 4 work on their run of key blocks as on a call of those keys alone
+  // (key 0 and the causal offset moved to the run's first key)
+  const int key_lo = C::split ? split * a.bps * kPfBN : 0;
+  const int Tk = C::split ? max(0, min(a.Tk - key_lo, a.bps * kPfBN)) : a.Tk;
   const int bhn = a.B * a.Hkv;
   const int hgrp = fdiv(u, a.dBH);
   const int bh = u - hgrp * bhn;
@@ -456,7 +478,7 @@ void prefill_fwd(const PrefillArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int l32 = lane & 31, h = lane >> 5;
-  const int off = a.Tk - a.Tq;                           // bottom-right causal offset
+  const int off = a.Tk - a.Tq - key_lo;                  // bottom-right causal offset
   // This wave's head (wave % hpw) and 32-row group (wave / hpw) of the
   // work-group's rpg = NW / hpw row groups per head.  With 8 waves, waves w
   // and w + 4 share a SIMD; under a causal mask later row groups see more key
@@ -487,18 +509,18 @@ void prefill_fwd(const PrefillArgs a) {
     }
   };
 
-  const int kend = a.causal ? min(a.Tk, off + q0 + 32 * rpg) : a.Tk;
+  const int kend = a.causal ? min(Tk, off + q0 + 32 * rpg) : Tk;
   const int nblk = kend > 0 ? (kend + kPfBN - 1) / kPfBN : 0;   // key blocks of the work-group
   const int wrow0 = q0 + rg * 32;                        // this wave's first row
-  const int wend = a.causal ? min(a.Tk, off + wrow0 + 32) : a.Tk;   // keys this wave can see
+  const int wend = a.causal ? min(Tk, off + wrow0 + 32) : Tk;   // keys this wave can see
   const int wblk = wend > 0 ? min(nblk, (wend + kPfBN - 1) / kPfBN) : 0;   // blocks this wave computes
   // blocks [0, wfull) are visible to every row of the wave: no mask
-  const int lim_all = a.causal ? min(a.Tk - 1, off + wrow0) : a.Tk - 1;
+  const int lim_all = a.causal ? min(Tk - 1, off + wrow0) : Tk - 1;
   const int wfull = lim_all >= 0 ? (lim_all + 1) / kPfBN : 0;
-  const int lim = a.causal ? min(a.Tk - 1, off + qi) : a.Tk - 1;   // this lane's last visible key
+  const int lim = a.causal ? min(Tk - 1, off + qi) : Tk - 1;   // this lane's last visible key
 
-  const char* kb = a.k + b * a.k_sb + (int64_t)hkv * a.k_sh;
-  const char* vimg = a.vimg + ((int64_t)b * a.Hkv + hkv) * a.nkb * VB;
+  const char* kb = a.k + b * a.k_sb + (int64_t)hkv * a.k_sh + (int64_t)key_lo * a.k_sn;
+  const char* vimg = a.vimg + (((int64_t)b * a.Hkv + hkv) * a.nkb + (C::split ? split * a.bps : 0)) * VB;
   // K stages are row-major with an XOR swizzle: 16-byte chunk c of key row r
   // sits in slot c ^ (r % NC) of the row's RB bytes.  A DMA instruction then
   // reads whole rows (16 lanes per 256-byte row at D = 128: coalesced), and
@@ -527,7 +549,7 @@ void prefill_fwd(const PrefillArgs a) {
     else if constexpr (NC == 8) return 4 * ((r >> 1) & 1);
     else return 0;
   };
-  const char* vb = kRawV ? a.v + b * a.v_sb + (int64_t)hkv * a.v_sh : nullptr;
+  const char* vb = kRawV ? a.v + b * a.v_sb + (int64_t)hkv * a.v_sh + (int64_t)key_lo * a.v_sn : nullptr;
   int v_voff[NK];
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
@@ -613,7 +635,7 @@ void prefill_fwd(const PrefillArgs a) {
   auto issue_k1 = [&](int blk, char* LK, int i) {
     const bool live = blk < nblk;
     const int key0 = live ? blk * kPfBN : 0;
-    const int rows = live ? min(kPfBN, a.Tk - key0) : 0;
+    const int rows = live ? min(kPfBN, Tk - key0) : 0;
     {
       const int c = wave * NK + i;
       const bool real = c < C::kdma;
@@ -631,7 +653,7 @@ void prefill_fwd(const PrefillArgs a) {
     const bool live = blk < nblk;
     if constexpr (kRawV) {
       const int key0 = live ? blk * kPfBN : 0;
-      const int rows = live ? min(kPfBN, a.Tk - key0) : 0;
+      const int rows = live ? min(kPfBN, Tk - key0) : 0;
       const int c = wave * NK + i;
       const bool real = c < C::kdma;
       const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
@@ -916,7 +938,7 @@ void prefill_fwd(const PrefillArgs a) {
   // whose second half lies past the wave's rows, or a ragged last block), the
   // second key tile's weights are all zero and its exponentials and PV MFMAs
   // are skipped.  Its V stage is picked at run time (one block per group).
-  const int wlim = a.causal ? min(a.Tk - 1, off + wrow0 + 31) : a.Tk - 1;   // the wave's last visible key
+  const int wlim = a.causal ? min(Tk - 1, off + wrow0 + 31) : Tk - 1;   // the wave's last visible key
   auto work_last = [&](const char* Vstage, int j, const f32x16& sa0, const f32x16& sa1) {
     if (j >= wblk) return;
     raise_max(rmax);
@@ -1110,7 +1132,21 @@ void prefill_fwd(const PrefillArgs a) {
   // chunks swizzled by row) so that every global store writes whole rows.
   wait_vmcnt<0>();                                         // every ring transfer (empty ones fill zeros) landed
   ring_barrier();                                        // every wave is done with the ring
-  {
+  if constexpr (C::split) {
+    // this run's fp32 partial (a row that sees none of its keys: max -inf, sum and O zero)
+    const float lt = half_swap_sum(l);
+    if (qi < a.Tq) {
+      const int64_t row = split * a.nrows + ((int64_t)b * a.Hq + hq) * a.Tq + qi;
+      float* dst = a.part_o + row * D + 4 * h;
+#pragma unroll
+      for (int e = 0; e < ET; ++e)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)
+          *(f32x4*)(dst + 32 * e + 8 * g4) =
+              f32x4{o[e][4 * g4], o[e][4 * g4 + 1], o[e][4 * g4 + 2], o[e][4 * g4 + 3]};
+      if (h == 0) *(float2*)(a.part_ml + 2 * row) = float2{m, lt};
+    }
+  } else {
     constexpr int NCH = D / 8;                           // 16-byte chunks per row
     char* tile = (wave >> 1) == 0 ? lk0 : (wave >> 1) == 1 ? lk1 : (wave >> 1) == 2 ? lk2 : lk3;
     tile += (wave & 1) * 32 * RB;
@@ -1137,6 +1173,55 @@ void prefill_fwd(const PrefillArgs a) {
         *(u32x4*)(a.out + b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)qrow * a.o_sm + c * 16) = w;
     }
   }
+}
+
+// Merge the nsplit partials of every output row (variants 3 and 4): D/4 lanes
+// per row, 4 dimensions each, so a wave reads whole 1 KB runs of consecutive
+// rows.  Batches of kMergeBatch runs are loaded together: the merge is a few
+// dependent round trips over data that L2 and the MALL hold (200 rows x 32
+// heads x 8 runs, 26 MB at head_dim 128: 6.1 us; 4 runs 4.9 us).
+constexpr int kMergeBatch = 8;
+
+template <int D, class T>
+__global__ __launch_bounds__(256) void prefill_merge(const PrefillArgs a) {
+  constexpr int LPR = D / 4, RPB = 256 / LPR;
+  const int li = threadIdx.x % LPR;
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  if (row >= a.nrows) return;
+  float M = -INFINITY, L = 0.f;
+  f32x4 A = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < a.nsplit; s0 += kMergeBatch) {
+    float2 ml[kMergeBatch];
+    f32x4 x[kMergeBatch];
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) {
+      const int64_t r = min(s0 + k, a.nsplit - 1) * a.nrows + row;   // (past the last run: reread, weighed out)
+      ml[k] = *(const float2*)(a.part_ml + 2 * r);
+      x[k] = *(const f32x4*)(a.part_o + r * D + 4 * li);
+    }
+    float mb = M;
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) {
+      if (s0 + k >= a.nsplit) ml[k].x = -INFINITY;
+      mb = fmaxf(mb, ml[k].x);
+    }
+    const float mref = mb == -INFINITY ? 0.f : mb;    // (no key seen yet: every weight is 2^-inf = 0)
+    const float r0 = fast_exp2(M - mref);
+    L *= r0;
+    A *= r0;
+#pragma unroll
+    for (int k = 0; k < kMergeBatch; ++k) {
+      const float w = fast_exp2(ml[k].x - mref);
+      L += w * ml[k].y;
+      A += w * x[k];
+    }
+    M = mb;
+  }
+  const float inv = L == 0.f ? 0.f : 1.0f / L;
+  const int bh = fdiv((int)row, a.dTq), qi = (int)row - bh * a.Tq;
+  const int b = fdiv(bh, a.dHq), hq = bh - b * a.Hq;
+  *(u32x2*)(a.out + b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)qi * a.o_sm + 8 * li) =
+      u32x2{pack2(T{}, A[0] * inv, A[1] * inv), pack2(T{}, A[2] * inv, A[3] * inv)};
 }
 
 }  // namespace sia

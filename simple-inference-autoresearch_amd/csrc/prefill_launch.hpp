@@ -11,7 +11,8 @@ struct PrefillLaunch {
   int D;
   int dtype;
   int var;         // prefill_fwd configuration: 0, or 1 = 4-wave groups at D = 128 (grids too small for the CUs),
-                   // 2 = variant 1 with the V^T images built in LDS (short key ranges; no prefill_pack_v)
+                   // 2 = variant 1 with the V^T images built in LDS (short key ranges; no prefill_pack_v),
+                   // 3 and 4 = key blocks split over work-groups (head_dim 64, 128 and 256; prefill_split.hip)
   hipStream_t stream;
 };
 
@@ -30,5 +31,12 @@ constexpr int kPackvMaxKeys = 512;
 constexpr int kPackvMaxKeysD64 = 768;
 
 int launch_prefill(PrefillLaunch& L);
+// Variants 3 and 4: prefill_fwd over runs of key blocks, then prefill_merge (called by launch_prefill).
+int launch_prefill_split(PrefillLaunch& L);
+
+// Rotary variant: none, or split-half / interleaved pairs from 16-bit / fp32 tables.
+inline int rope_variant(const PrefillArgs& a) {
+  return a.cs == nullptr ? kRopeNone : 1 + (a.interleaved ? 1 : 0) + (a.tab_dt == SIA_F32 ? 2 : 0);
+}
 
 }  // namespace sia

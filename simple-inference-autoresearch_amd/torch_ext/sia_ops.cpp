@@ -188,16 +188,6 @@ Tensor readable(const Tensor& t) {
   return ok ? t : t.contiguous();
 }
 
-// The prefill takes no workspace for fp32 (vector-ALU path) and for float16
-// at head_dim 32-128, whose V is read in place; otherwise V is repacked into
-// f16 block images in the workspace.  (The same rule as v_in_place in
-// csrc/capi_prefill.cpp; were they to differ, the library would refuse the
-// call with SIA_ERR_WORKSPACE rather than touch memory it was not given.)
-bool v_in_place(const Tensor& q) {
-  const int64_t D = q.size(-1);
-  return q.scalar_type() == at::kFloat || (q.scalar_type() == at::kHalf && D >= 32 && D <= 128);
-}
-
 // Causal / full attention (q (B, Hq, Tq, D)) -> (B, Hq, Tq, D) or token-major (B, Tq, Hq, D).
 Tensor prefill(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, bool causal, double sm_scale,
                bool out_token_major) {
@@ -212,7 +202,7 @@ Tensor prefill(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, bool 
   const Tensor view = out_token_major ? out.transpose(1, 2) : out;
   const sia_tensor dout = desc(view, dev, "out");
   size_t ws_bytes = 0;
-  if (!v_in_place(q)) check(sia_prefill_workspace_size(B, Hkv, Tk, D, &ws_bytes));
+  check(sia_attention_flash_fwd_workspace_size(&dq, &dk, &ws_bytes));
   Tensor ws = ws_bytes > 0 ? at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte)) : Tensor();
   check(sia_attention_flash_fwd(&dq, &dk, &dv, causal ? 1 : 0, (float)sm_scale, &dout,
                                 ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(dev)));
@@ -236,7 +226,7 @@ Tensor prefill_rope(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, 
   const Tensor view = out_token_major ? out.transpose(1, 2) : out;
   const sia_tensor dout = desc(view, dev, "out");
   size_t ws_bytes = 0;
-  if (!v_in_place(q)) check(sia_prefill_workspace_size(B, Hkv, Tk, D, &ws_bytes));
+  check(sia_attention_flash_fwd_workspace_size(&dq, &dk, &ws_bytes));
   Tensor ws = ws_bytes > 0 ? at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte)) : Tensor();
   check(sia_attention_flash_fwd_rope(&dq, &dk, &dv, &dc, &dsn, interleaved ? 1 : 0, dsp.ptr(), (int32_t)start_offset,
                                      causal ? 1 : 0, (float)sm_scale, &dout, ws_bytes > 0 ? ws.data_ptr() : nullptr,
