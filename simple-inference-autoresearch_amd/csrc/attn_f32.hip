@@ -78,27 +78,15 @@ __global__ __launch_bounds__(256) void attn_f32(const F32Args a) {
   const int hkv = item % a.Hkv;
   const int b = item / a.Hkv;
 
-  // columns of this item: keys visible to each, and the query slice
-  int n_all = a.cap;
-  if (a.kv_len != nullptr) {
-    const int n = a.kv_len[a.kv_per_seq ? b : 0];
-    n_all = n < 0 ? 0 : (n > a.cap ? a.cap : n);
-  }
-  int lim[C];
+  // the sequence's keys, and the query slice of every column
+  const int n = a.kv_len[a.kv_per_seq ? b : 0];
+  const int nmax = n < 0 ? 0 : (n > a.cap ? a.cap : n);
   f32x4 q[C];
-  int nmax = 0;
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    const int col = chunk * C + c;
-    const bool live = col < a.ncol;
-    const int i = live ? col / a.G : 0;
-    const int g = live ? col - i * a.G : 0;
-    int n = live ? n_all : 0;
-    if (a.causal) n = min(n, a.Tk - a.Tq + i + 1);
-    lim[c] = n > 0 ? n : 0;
-    nmax = max(nmax, lim[c]);
-    const char* qp = a.q + b * a.q_sb + (int64_t)(hkv * a.G + g) * a.q_sh + (int64_t)i * a.q_sm +
-                     j4 * 4 * QT::bytes;
+    const int g = chunk * C + c;                          // column: query head g of the KV head's group
+    const bool live = g < a.ncol;
+    const char* qp = a.q + b * a.q_sb + (int64_t)(hkv * a.G + (live ? g : 0)) * a.q_sh + j4 * 4 * QT::bytes;
     q[c] = live ? load4<QT>(qp) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int lo = s * a.tps;
@@ -165,7 +153,7 @@ __global__ __launch_bounds__(256) void attn_f32(const F32Args a) {
         for (int o = LPT / 2; o > 0; o >>= 1) d += __shfl_xor(d, o);
         if constexpr (kInt8) d *= ksc[u];
         d *= a.qk_scale;
-        sc[u] = tt[u] < hi && tt[u] < lim[c] ? d : -INFINITY;
+        sc[u] = tt[u] < hi ? d : -INFINITY;
       }
       float smax = sc[0];
 #pragma unroll
@@ -218,14 +206,13 @@ __global__ __launch_bounds__(256) void attn_f32(const F32Args a) {
     f32x4 A = *(const f32x4*)&sm[0][c][4 * jj];
 #pragma unroll
     for (int w = 1; w < 4; ++w) merge_state(M, L, A, sm[w][c][D], sm[w][c][D + 1], *(const f32x4*)&sm[w][c][4 * jj]);
-    const int i = col / a.G, g = col - i * a.G;
-    const int hq = hkv * a.G + g;
+    const int hq = hkv * a.G + col;
     if (a.nsplit == 1) {
       const float inv = L == 0.f ? 0.f : 1.0f / L;     // no visible key: zeros (the reference's l_safe guard)
-      char* op = a.out + b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)i * a.o_sm + jj * 4 * QT::bytes;
+      char* op = a.out + b * a.o_sb + (int64_t)hq * a.o_sh + jj * 4 * QT::bytes;
       store4(QT{}, op, A * inv);
     } else {
-      const int64_t row = ((int64_t)b * a.Hq + hq) * a.Tq + i;
+      const int64_t row = (int64_t)b * a.Hq + hq;
       float* dst = a.part + (row * a.nsplit + s) * (D + 4);
       *(f32x4*)(dst + 4 * jj) = A;
       if (jj == 0) {
@@ -243,7 +230,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
   const int lane = threadIdx.x & 63;
   const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPT;
   const int jj = lane % LPT;
-  if (row >= (int64_t)a.B * a.Hq * a.Tq) return;
+  if (row >= (int64_t)a.B * a.Hq) return;
   const float* p = a.part + row * a.nsplit * (D + 4);
   float M = -INFINITY;
   for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, p[s * (D + 4) + D]);
@@ -257,12 +244,10 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
       A += w * *(const f32x4*)(p + s * (D + 4) + 4 * jj);
     }
   }
-  const int i = (int)(row % a.Tq);
-  const int64_t bh = row / a.Tq;
-  const int hq = (int)(bh % a.Hq);
-  const int b = (int)(bh / a.Hq);
+  const int b = (int)(row / a.Hq);
+  const int hq = (int)(row - (int64_t)b * a.Hq);
   const float inv = L == 0.f ? 0.f : 1.0f / L;
-  store4(OT{}, a.out + b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)i * a.o_sm + jj * 4 * OT::bytes, A * inv);
+  store4(OT{}, a.out + b * a.o_sb + (int64_t)hq * a.o_sh + jj * 4 * OT::bytes, A * inv);
 }
 
 template <int D, class QT, class KV, class ST>
@@ -281,7 +266,7 @@ static int launch_f32_typed(F32Launch& L) {
   }
   if (a.nsplit > 1) {
     constexpr int RPB = 4 * (64 / (D / 4));
-    const int64_t rows = (int64_t)a.B * a.Hq * a.Tq;
+    const int64_t rows = (int64_t)a.B * a.Hq;
     const int64_t blocks = (rows + RPB - 1) / RPB;
     if (blocks > 0x7fffffff) return fail(SIA_ERR_UNSUPPORTED, "fp32 attention: too many rows");
     hipLaunchKernelGGL((attn_f32_merge<D, QT>), dim3((unsigned)blocks), dim3(256), 0, L.stream, a);
@@ -306,7 +291,7 @@ static int launch_f32_d(F32Launch& L) {
 template <int D>
 static int launch_merge_d(const F32Args& a, int out_dtype, hipStream_t st) {
   constexpr int RPB = 4 * (64 / (D / 4));
-  const int64_t rows = (int64_t)a.B * a.Hq * a.Tq;
+  const int64_t rows = (int64_t)a.B * a.Hq;
   const int64_t blocks = (rows + RPB - 1) / RPB;
   if (blocks > 0x7fffffff) return fail(SIA_ERR_UNSUPPORTED, "split-K merge: too many rows");
   if (blocks == 0) return SIA_OK;

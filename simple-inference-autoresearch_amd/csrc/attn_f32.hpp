@@ -1,22 +1,18 @@
-// Float32 attention on the vector ALUs: the path for calls whose q or K/V are
-// float32 (decode and prefill).
+// Float32 attention: decode calls whose q or K/V are float32 (attn_f32, on
+// the vector ALUs), and prefill in float32 (attn_f32_prefill.hip, fp32 MFMAs).
 //
 // The reference wrappers accept any float dtype and return q's dtype
 // (kernels/flash_decode_kernel.py:119-160, kernels/attention_kernel.py:235-305);
 // its decode kernel computes in fp32 on vector lanes, tl.sum(q * k) and
 // tl.sum(p * v) with an online softmax (kernels/flash_decode_kernel.py:85-114).
-// The MFMA kernels of this library take 16-bit or int8 operands, so float32
-// inputs run here instead, in fp32 end to end: products, sums, exponentials
-// and the output (rounded to q's dtype).
+// The 16-bit MFMA kernels of this library take 16-bit or int8 operands, so
+// float32 inputs run here instead, in fp32 end to end: products, sums,
+// exponentials and the output (rounded to q's dtype).
 //
-// Layout (gfx950, wave64):
-//  * A work item is one (sequence, KV head), up to kF32Cols "columns" -- the
-//    (query row, query head) pairs of that KV head -- and one split of the
-//    key range.  The K/V rows of the item are read once for all of its
-//    columns (GQA: the G query heads of a KV head; prefill: several query
-//    rows too).  Column (i, g) sees keys [0, n_i): n = kv_len (decode) or
-//    Tk, and with the causal mask n_i = min(n, Tk - Tq + i + 1) (bottom-right,
-//    kernels/attention_kernel.py:184-226); n_i <= 0 writes zeros.
+// attn_f32 (gfx950, wave64):
+//  * A work item is one (sequence, KV head), up to kF32Cols of its query heads
+//    ("columns") and one split of the key range [0, kv_len).  The K/V rows of
+//    the item are read once for all of its columns.
 //  * D/4 lanes share a key row, 4 dimensions each (16-byte fp32 loads; 8 or 4
 //    bytes for 16-bit and int8 K/V), so one load instruction of a wave reads
 //    64/(D/4) whole rows.  Each lane group runs an online softmax over its
@@ -33,7 +29,8 @@
 
 namespace sia {
 
-constexpr int kF32Cols = 8;     // columns (query row, head) per work item
+constexpr int kF32Cols = 8;     // columns (query heads) per work item of attn_f32
+constexpr int kF32TileCols = 32;   // columns per work-group of the prefill kernel (attn_f32_prefill.hip)
 constexpr int kF32Unroll = 4;   // keys per lane group per step
 
 struct F32Args {
@@ -46,11 +43,12 @@ struct F32Args {
   const int32_t* bt; int64_t bt_sb, bt_sl;           // block table (element strides), nullptr = contiguous
   int64_t num_pages;
   int32_t page_size;
-  const int32_t* kv_len; int32_t kv_per_seq;         // nullptr: every column sees `cap` keys (prefill)
-  int32_t cap;                                       // keys addressable: S, max_blocks * page_size, or Tk
+  const int32_t* kv_len; int32_t kv_per_seq;         // (decode)
+  int32_t cap;                                       // keys addressable: S or max_blocks * page_size (decode)
   int32_t B, Hq, Hkv, G, Tq, Tk, causal;
   int32_t ncol;                                      // Tq * G columns per (sequence, KV head)
-  int32_t nchunk;                                    // ceil(ncol / kF32Cols)
+  int32_t nchunk;                                    // ceil(ncol / columns per work item)
+  int32_t fold;                                      // prefill kernel: CU count, or 0 (see there)
   int32_t nsplit, tps;                               // key-range split: nsplit pieces of tps keys
   float qk_scale;                                    // sm_scale * log2(e)
   float* part;                                       // nsplit > 1: [row][split][D + 4] (acc, m, l)
@@ -69,6 +67,10 @@ struct F32Launch {
 
 // Launches attn_f32 (and attn_f32_merge when nsplit > 1); implemented in attn_f32.hip.
 int launch_attn_f32(F32Launch& L);
+
+// Prefill of float32 q, k, v on the matrix cores: nchunk = ceil(ncol /
+// kF32TileCols), no split, no paging (attn_f32_prefill.hip).
+int launch_attn_f32_prefill(F32Launch& L);
 
 // attn_f32_merge alone, for split-K partials written in its layout by another
 // kernel: head_dim D, output dtype out_dtype (f16 / bf16 / f32).

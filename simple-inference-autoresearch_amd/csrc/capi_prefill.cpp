@@ -99,8 +99,8 @@ KeySplit key_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, 
   return best;
 }
 
-// Float32 q/k/v: the vector-ALU path (attn_f32.hpp), one work item per
-// (sequence, KV head, chunk of query rows x heads), no workspace.
+// Float32 q/k/v: fp32 MFMAs (attn_f32_prefill.hip), one work-group per
+// (sequence, KV head, 32 query rows x heads), no workspace.
 int prefill_f32(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int32_t causal, float sm_scale,
                 const sia_tensor* out, void* stream) {
   const int64_t B = q->shape[0], Hq = q->shape[1], Tq = q->shape[2], D = q->shape[3];
@@ -122,15 +122,13 @@ int prefill_f32(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, i
   a.B = (int)B; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)G; a.Tq = (int)Tq; a.Tk = (int)Tk;
   a.causal = causal != 0;
   a.ncol = (int)(Tq * G);
-  a.nchunk = (int)((Tq * G + kF32Cols - 1) / kF32Cols);
-  a.nsplit = 1;
-  a.tps = Tk > 0 ? (int)Tk : 1;
+  a.nchunk = (int)((Tq * G + kF32TileCols - 1) / kF32TileCols);
   a.qk_scale = sm_scale * 1.4426950408889634f;
   L.D = (int)D;
   L.q_dtype = SIA_F32;
   L.kv_dtype = SIA_F32;
   L.stream = (hipStream_t)stream;
-  return launch_attn_f32(L);
+  return launch_attn_f32_prefill(L);
 }
 
 // Rotary tables of the fused entry point (NULL cos: no rotation).
