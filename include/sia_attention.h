@@ -180,8 +180,8 @@ int sia_paged_gqa_int8_flash_decode_noalloc(const sia_tensor* q, const sia_tenso
  * layout (float16 V at head_dim 32-128 needs none: NULL, 0 is accepted
  * there) and is free again when the stream passes the call.  With
  * sia_attention_flash_fwd_workspace_size bytes a call of few query rows over
- * many keys may also split its keys.  f32 inputs run in fp32 on the fp32
- * ALUs and need no workspace (NULL, 0 is accepted). */
+ * many keys may also split its keys.  f32 inputs run in fp32 on the
+ * matrix cores and need no workspace (NULL, 0 is accepted). */
 int sia_attention_flash_fwd(const sia_tensor* q, const sia_tensor* k, const sia_tensor* v, int32_t causal,
                             float sm_scale, const sia_tensor* out, void* workspace, size_t workspace_bytes,
                             void* stream);

@@ -67,6 +67,8 @@ struct DecodeArgs {
   int32_t cap_tokens;                                // S (contiguous) or max_blocks*page_size
   int32_t B, Hq, Hkv, G, HG, U, UB;                  // U = Hkv*HG units per sequence, UB unit blocks per item row
   int32_t IU;                                        // units per item (NW / IU waves per unit)
+  int32_t lgP;                                       // log2 of the waves per unit
+  FastDiv dHG, dUB, dHq, dG, dIU;                    // divisions by HG, UB, Hq, G, IU
   float qk_scale;                                    // sm_scale * log2(e)
   float* ws_acc; float* ws_ml; int32_t* ws_plan; int32_t max_items; int32_t G16;
   int32_t tps_force;
@@ -148,13 +150,35 @@ template <int NW>
 __device__ int plan_work(const DecodeArgs& a, int* pre, int* red, int tok0, int& pen) {
   const int T = NW * 64;
   if (!a.kv_per_seq) {
-    pen = 0;
-    const int per = ((tok0 + kTile - 1) / kTile) * a.UB;
-    for (int b = threadIdx.x; b <= a.B; b += T) pre[b] = b * per;
-    __syncthreads();
-    return a.B * per;
+    pen = 0;   // (no prefix in LDS: seg_at has the closed form)
+    return a.B * (((tok0 + kTile - 1) / kTile) * a.UB);
   }
   int* lens = pre + a.B + 1;                 // token counts, kept for the segments (small batches)
+  if (a.B <= 64) {
+    // one length per lane: every wave scans by itself, the first one leaves
+    // the prefix in LDS (one barrier instead of the block-wide scan's four:
+    // with it 2.2 us of a group's start at 8 sequences)
+    const int lane = threadIdx.x & 63;
+    const int n = lane < a.B ? seq_tokens(a, lane) : 0;
+    const int nt = (n + kTile - 1) / kTile;
+    pen = __all(lane >= a.B || nt == uniform(nt)) ? 0 : a.seg_pen;
+    const int w = (nt + (nt > 0 ? pen : 0)) * a.UB;
+    int incl = w;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    if (threadIdx.x < 64) {
+      if (lane < a.B) {
+        pre[lane] = incl - w;
+        lens[lane] = n;
+      }
+      if (lane == 63) pre[a.B] = incl;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readlane(incl, 63);
+  }
   int nmin = 0x7fffffff, nmax = -1;
   for (int b = threadIdx.x; b < a.B; b += T) {
     const int n = seq_tokens(a, b);
@@ -179,15 +203,44 @@ __device__ int plan_work(const DecodeArgs& a, int* pre, int* red, int tok0, int&
   // taken as divergent and every tile load wrapped in a waterfall loop)
   pen = uniform(nmin == nmax ? 0 : a.seg_pen);
   block_scan<NW>(a, pre, red, a.UB, pen);
-  return pre[a.B];
+  return uniform(pre[a.B]);
 }
 
 // Stream-K split of W tiles over G work-groups: group g takes
-// [lo(g), lo(g+1)) with lo(g) = floor(g W / G); the group holding position x
-// is ceil((x+1) G / W) - 1.
-__device__ __forceinline__ int sk_lo(int g, int W, int G) { return (int)((int64_t)g * W / G); }
-__device__ __forceinline__ int sk_group(int x, int W, int G) {
-  return (int)(((int64_t)(x + 1) * G + W - 1) / W) - 1;
+// [lo(g), lo(g+1)) with lo(g) = floor(g W / G).  With W = Q G + R this is
+// g Q + floor(g R / G), and g R < G^2 (G is at most the persistent grid, some
+// thousand) stays below 2^24, where one fp32 product and a correction divide
+// exactly.  (The 64-bit divisions this replaces took ~0.4 us of every group's
+// start at one sequence of 1000 tokens.)
+struct SkSplit {
+  int W, G, Q, R;
+  float rG;            // 1 / G
+};
+__device__ __forceinline__ SkSplit sk_split(int W, int G) {
+  SkSplit s;
+  s.W = W;
+  s.G = G;
+  s.Q = (int)((uint32_t)W / (uint32_t)G);
+  s.R = W - s.Q * G;
+  s.rG = __builtin_amdgcn_rcpf((float)G);
+  return s;
+}
+__device__ __forceinline__ int sk_lo(const SkSplit& s, int g) {
+  const int n = g * s.R;
+  int q = (int)((float)n * s.rG);
+  const int r = n - q * s.G;
+  q += r >= s.G ? 1 : r < 0 ? -1 : 0;
+  return g * s.Q + q;
+}
+// The group holding position x (0 <= x < W), the last one with lo(g) <= x:
+// ceil((x + 1) G / W) - 1 by an fp32 estimate, within one of it (the error is
+// below G 2^-21), set right by the bounds.
+__device__ __forceinline__ int sk_group(const SkSplit& s, int x) {
+  int g = (int)ceilf((float)(x + 1) * ((float)s.G * __builtin_amdgcn_rcpf((float)s.W))) - 1;
+  g = min(max(g, 0), s.G - 1);
+  if (g > 0 && sk_lo(s, g) > x) --g;
+  if (g + 1 < s.G && sk_lo(s, g + 1) <= x) ++g;
+  return g;
 }
 
 // -------------------------------------------------------------- tile data
@@ -602,8 +655,25 @@ template <int NW>
 __device__ __forceinline__ ItemShape item_shape(const DecodeArgs& a) {
   ItemShape sh;
   sh.units = a.IU;
-  sh.P = NW / a.IU;
+  sh.P = 1 << a.lgP;
   return sh;
+}
+
+// Groups for one shared length of nt tiles: the equal shares of G groups
+// generally straddle segment boundaries, and a group that holds the end of
+// one segment and the start of the next pays the start chain (length, query,
+// page id, first tile) and the merge twice, ~6 us.  A multiple of the segment
+// count gives every group one piece of one segment instead, at the cost of
+// the groups left over: taken when those cost less.  (B8 x 1000 tokens, 64
+// segments on 248 groups: 56 groups ended 8 us after the others.)
+__device__ __forceinline__ int aligned_groups(const DecodeArgs& a, int nt, int G, int P, int row_bytes) {
+  const int nseg = a.B * a.UB;
+  if (G <= nseg) return G;
+  const int S = (int)((uint32_t)G / (uint32_t)nseg), G1 = nseg * S;
+  // tiles a wave gains, times ~1.3 us per 4 KB of K and V tile (every CU streaming)
+  const float more = (float)nt * ((float)nseg * __builtin_amdgcn_rcpf((float)P)) *
+                     (__builtin_amdgcn_rcpf((float)G1) - __builtin_amdgcn_rcpf((float)G));
+  return uniform(more * (float)row_bytes * (1.3f / 128.0f) < 6.0f) ? G1 : G;
 }
 
 template <int D, class KV, class QT, class ST, int NW, bool SV>
@@ -635,8 +705,11 @@ void decode_main(const DecodeArgs a) {
   // segments on one group took ~50 us)
   G = min(G, max(a.B * a.UB, (W + kMinWaveTiles * shape.P - 1) / (kMinWaveTiles * shape.P)));
   G = min(G, max(1, a.max_items / 2));                      // two partial slots per group
+  const int nt0 = (tok0 + kTile - 1) / kTile;               // (one shared length)
+  if (!a.kv_per_seq && a.tps_force <= 0) G = aligned_groups(a, nt0, G, shape.P, KV::bytes * D);
   if (blockIdx.x == 0) {
-    for (int i = threadIdx.x; i <= a.B; i += NW * 64) a.ws_plan[kPlanHeader + i] = pre[i];
+    for (int i = threadIdx.x; i <= a.B; i += NW * 64)
+      a.ws_plan[kPlanHeader + i] = a.kv_per_seq ? pre[i] : i * nt0 * a.UB;
     if (threadIdx.x == 0) {
       a.ws_plan[kPlanW] = W;
       a.ws_plan[kPlanG] = G;
@@ -657,8 +730,10 @@ void decode_main(const DecodeArgs a) {
     return;
   }
   const int g = blockIdx.x;
-  const int x_hi = g < G ? sk_lo(g + 1, W, G) : 0;
-  int x = g < G ? sk_lo(g, W, G) : 0;
+  if (g >= G) return;                                       // (the whole work-group)
+  const SkSplit sk = sk_split(W, G);
+  const int x_hi = sk_lo(sk, g + 1);
+  int x = sk_lo(sk, g);
   int* prog = red + 2;   // tiles done per wave (NW ints; read and written without barriers)
 
   const int lane = threadIdx.x & 63;
@@ -671,8 +746,8 @@ void decode_main(const DecodeArgs a) {
   for (int i = 0; i < 4; ++i) lo.v[i] = (4 * grp + i) * a.v_tok + (uint32_t)(lane16 * (TileT::kVSplit ? 16 : TileT::VB));
   lo.ks = 4 * grp * a.ks_tok;
   lo.vs = 4 * grp * a.vs_tok;
-  const int uin = wave / shape.P;        // unit slot of this wave inside an item
-  const int phase = wave - uin * shape.P;
+  const int uin = wave >> a.lgP;         // unit slot of this wave inside an item
+  const int phase = wave & (shape.P - 1);
 
   // Segments: the maximal pieces of [x, x_hi) inside one (sequence, unit
   // block).  A segment that covers its whole (b, ublk) is written straight to
@@ -690,16 +765,34 @@ void decode_main(const DecodeArgs a) {
   };
   auto seg_at = [&](int xs) {
     SegAt s;
-    int blo = 0, bhi = a.B;
-    while (bhi - blo > 1) { const int mid = (blo + bhi) >> 1; if (pre[mid] <= xs) blo = mid; else bhi = mid; }
-    s.b = uniform(blo);
-    s.ntok = a.kv_per_seq ? uniform(a.B <= kLensInLds ? pre[a.B + 1 + s.b] : seq_tokens(a, s.b)) : tok0;
-    s.ntile = (s.ntok + kTile - 1) / kTile;
+    int pb;
+    if (!a.kv_per_seq) {
+      s.ntok = tok0;
+      s.ntile = nt0;
+      const int sidx = (int)((uint32_t)xs / (uint32_t)nt0);  // (xs < W: nt0 > 0)
+      s.b = uniform(fdiv(sidx, a.dUB));
+      pb = s.b * nt0 * a.UB;
+    } else {
+      // the largest b with pre[b] <= xs: counted 64 entries at a time, from
+      // the block of the coarse search on (a binary search reads LDS once per
+      // step, ~60 ns each)
+      int base = 0;
+      for (int n = a.B; n > 64;) {
+        const int half = n >> 1;
+        if (pre[base + half] <= xs) { base += half; n -= half; }
+        else n = half;
+      }
+      const int i = base + lane;
+      s.b = base + __popcll(__ballot(i < a.B && pre[i] <= xs)) - 1;
+      s.ntok = uniform(a.B <= kLensInLds ? pre[a.B + 1 + s.b] : seq_tokens(a, s.b));
+      s.ntile = (s.ntok + kTile - 1) / kTile;
+      pb = uniform(pre[s.b]);
+    }
     const int nvt = s.ntile + pen;
-    const int rem = uniform(xs - pre[s.b]);
-    s.ublk = rem / nvt;
+    const int rem = uniform(xs) - pb;
+    s.ublk = a.UB == 1 ? 0 : (int)((uint32_t)rem / (uint32_t)nvt);
     const int r_lo = rem - s.ublk * nvt;
-    s.seg_end = min(x_hi, pre[s.b] + (s.ublk + 1) * nvt);
+    s.seg_end = min(x_hi, pb + (s.ublk + 1) * nvt);
     const int r_hi = r_lo + (s.seg_end - xs);
     s.t_lo = max(0, r_lo - pen);
     s.t_hi = max(0, r_hi - pen);
@@ -708,6 +801,9 @@ void decode_main(const DecodeArgs a) {
   // The next segment's query row and first page id are loaded while the
   // current one streams (seg_next: the start of the segment they belong
   // to), so that a segment change waits for its first tile only.
+  // (Not where its registers do not fit: 16-bit K/V at head_dim 64 in 128
+  // registers, int8 with scattered scales.)
+  constexpr bool kNext = TileT::kInt8 ? SV : D > 64;
   QRaw<D> q_next;
   int pg_next = 0, seg_next = -1;
   bool first_seg = true;
@@ -723,7 +819,7 @@ void decode_main(const DecodeArgs a) {
     const int pslot_id = first_seg ? 2 * g : 2 * g + 1;
     const int unit = ublk * shape.units + uin;
     const bool wave_live = uin < shape.units && unit < a.U;
-    const int hkv = unit / a.HG, hg = unit - hkv * a.HG;
+    const int hkv = fdiv(unit, a.dHG), hg = unit - hkv * a.HG;
     const int nh = wave_live ? min(16, a.G - 16 * hg) : 0;    // live head columns of this wave's unit
     const bool live = lane16 < nh;
     const int hq = live ? hkv * a.G + 16 * hg + lane16 : 0;
@@ -745,15 +841,21 @@ void decode_main(const DecodeArgs a) {
       const int64_t bt_step = paged ? a.bt_sl : 0;
       const int cap_tiles = a.cap_tokens / kTile;
       auto page_id = [&](int k) {
+        if (!paged) return 0;      // (nothing to wait for)
         const int t = min(t_first + k * P, cap_tiles - 1);
         return uniform(btrow[(int64_t)(t >> a.lg_tiles_per_page) * bt_step]);
       };
-      // The loads that need only the item go out together: the query row
-      // and the first tile's page id (the length is already in flight),
-      // unless the previous segment loaded them already.
+      const int t_full = min(t_hi, ntok / kTile);
+      const int nfull = t_first < t_full ? (t_full - t_first + P - 1) >> a.lgP : 0;
+      const int nt = t_first < t_hi ? (t_hi - t_first + P - 1) >> a.lgP : 0;
+      // The loads that need only the item go out together: the query row and
+      // the page ids of the first tile and of the partial one (the length is
+      // already in flight), unless the previous segment loaded them already.
       QRaw<D> qraw;
       int pg0;
-      if (x == seg_next) {
+      constexpr bool kPartFirst = D > 64 || TileT::kInt8;   // (see below)
+      int pgl = kPartFirst && nt > nfull ? page_id(nfull) : 0;
+      if (kNext && x == seg_next) {
         qraw = q_next;
         pg0 = pg_next;
       } else {
@@ -763,11 +865,11 @@ void decode_main(const DecodeArgs a) {
       // the next segment of the share, if this wave has a unit there: its
       // query row and first page id (issued behind this segment's first tile)
       auto prefetch_next = [&]() {
-        if (seg_end >= x_hi) return;
+        if (!kNext || seg_end >= x_hi) return;
         const SegAt nx = seg_at(seg_end);
         const int unit_n = nx.ublk * shape.units + uin;
         if (nx.t_hi == nx.t_lo || unit_n >= a.U) return;
-        const int hkv_n = unit_n / a.HG, hg_n = unit_n - hkv_n * a.HG;
+        const int hkv_n = fdiv(unit_n, a.dHG), hg_n = unit_n - hkv_n * a.HG;
         const bool live_n = lane16 < min(16, a.G - 16 * hg_n);
         const int hq_n = live_n ? hkv_n * a.G + 16 * hg_n + lane16 : 0;
         q_next = load_q_raw<D, KV>(a, nx.b, hq_n, live_n, grp);
@@ -776,9 +878,6 @@ void decode_main(const DecodeArgs a) {
         pg_next = uniform(btrow_n[(int64_t)(tn >> a.lg_tiles_per_page) * bt_step]);
         seg_next = seg_end;
       };
-      const int t_full = min(t_hi, ntok / kTile);
-      const int nfull = t_first < t_full ? (t_full - t_first + P - 1) / P : 0;
-      const int nt = t_first < t_hi ? (t_hi - t_first + P - 1) / P : 0;
       const int64_t rowk = paged ? 0 : (int64_t)b * a.k_s0, rowv = paged ? 0 : (int64_t)b * a.v_s0;
       const int64_t rowks = paged ? 0 : (int64_t)b * a.ks_s0, rowvs = paged ? 0 : (int64_t)b * a.vs_s0;
       const char* kb = a.k + (rowk + (int64_t)hkv * a.k_sh);
@@ -806,14 +905,31 @@ void decode_main(const DecodeArgs a) {
       };
       u32x4 qop[KSTEPS], qop_lo[KSTEPS];
       float qmul = 0.f;
+      // The sequence's partial last tile, if it is this wave's, is loaded and
+      // computed first (its order is free), while the first full tile is in
+      // flight: behind the full tiles it was one more dependent round trip of
+      // the wave that every other wave of the unit waited for, 2 us at one
+      // sequence of 1000 tokens.  (16-bit K/V at head_dim 64 has no registers
+      // for it in its 128, spills cost 4-17%, and takes it last.)
+      const bool part = nt > nfull;
+      TileT last;
+      auto load_part = [&]() {
+        if (part)
+          load_tile<D, KV, ST, false, false>(a, tile_ptr(t_first + nfull * P, pgl), lo,
+                                             ntok - (t_first + nfull * P) * kTile, last, lane16, grp);
+      };
+      auto compute_part = [&]() {
+        if (part) compute_tile<D, KV, QT, ST, false>(last, qop, qop_lo, qmul, t_first + nfull * P, ntok, grp, st);
+      };
+      if constexpr (kPartFirst) load_part();
       // Full tiles, double-buffered.  The steady-state loop always issues the
       // next tiles' loads, and fetches the page ids of the tiles two ahead
       // with one vector load (lanes 0 and 1; indices clamped to the wave's
-      // last tile, the partial one included), so every load retires in order
-      // and computing tile k waits only for tile k.
-      int pg_last = pg0;   // page of the wave's partial last tile (tile nfull)
+      // last tile of them), so every load retires in order and computing tile k
+      // waits only for tile k.
+      if (!kPartFirst) pgl = pg0;
       if (nfull > 0) {
-        const int klast = nt > nfull ? nfull : nfull - 1;
+        const int klast = !kPartFirst && nt > nfull ? nfull : nfull - 1;
         auto page_pair = [&](int k0) {
           const int k = min(k0 + (lane & 1), klast);
           const int t = t_first + k * P;
@@ -827,6 +943,7 @@ void decode_main(const DecodeArgs a) {
         prefetch_next();
         // the query's conversion overlaps the first tile's flight
         qmul = prep_q<D, KV, QT>(a, qraw, qop, qop_lo);
+        if constexpr (kPartFirst) compute_part();
         int k = 0;
         for (; k + 2 < nfull; k += 2) {
           // With 8 waves, waves w and w^4 share a SIMD, where the older one
@@ -851,9 +968,9 @@ void decode_main(const DecodeArgs a) {
           __builtin_amdgcn_s_setprio(0);
           __hip_atomic_store(&prog[wave], 1 << 30, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        // pgv holds the pages of tiles k + 1 and k + 2 (clamped); the partial
-        // tile, if any, is tile nfull = k + 1 or k + 2
-        pg_last = __builtin_amdgcn_readlane(pgv, nfull - k - 1);
+        // (pgv holds the pages of tiles k + 1 and k + 2, clamped; the partial
+        // tile, taken last, is one of the two)
+        if constexpr (!kPartFirst) pgl = __builtin_amdgcn_readlane(pgv, nfull - k - 1);
         if (k + 1 < nfull) {
           load_tile<D, KV, ST, true, SV>(a, tile_ptr(t_first + (k + 1) * P, __builtin_amdgcn_readlane(pgv, 0)), lo,
                                          16, bufB, lane16, grp);
@@ -865,12 +982,11 @@ void decode_main(const DecodeArgs a) {
       } else {
         prefetch_next();
         qmul = prep_q<D, KV, QT>(a, qraw, qop, qop_lo);
+        if constexpr (kPartFirst) compute_part();
       }
-      if (nt > nfull) {  // the sequence's partial last tile belongs to this wave
-        const int t = t_first + nfull * P;
-        TileT last;
-        load_tile<D, KV, ST, false, false>(a, tile_ptr(t, pg_last), lo, ntok - t * kTile, last, lane16, grp);
-        compute_tile<D, KV, QT, ST, false>(last, qop, qop_lo, qmul, t, ntok, grp, st);
+      if constexpr (!kPartFirst) {
+        load_part();
+        compute_part();
       }
     }
 
@@ -906,7 +1022,12 @@ void decode_main(const DecodeArgs a) {
         }
       }
     } else {
-      // P waves per unit: merge their (m, l, acc) through LDS
+      // P waves per unit: merge their (m, l, acc) through LDS.  Wave `phase`
+      // of a unit finishes head columns phase, phase + P, ..., D / 64 elements
+      // per lane; the P states of a column are read together, so a column
+      // costs two LDS round trips.  (A flat loop over all elements, with the
+      // states read one after the other and three runtime divisions each, took
+      // 3.4 us of a 10.7 us group at one sequence of 1000 tokens.)
       if (live) {
         float* dst = l_acc + (wave * a.G16 + lane16) * D;
 #pragma unroll
@@ -919,37 +1040,56 @@ void decode_main(const DecodeArgs a) {
         l_l[wave * a.G16 + lane16] = live ? lsum : 0.f;
       }
       __syncthreads();
-      const int nh_all = min(16, a.G);                 // head columns per unit (same for every unit here)
-      for (int idx = threadIdx.x; idx < shape.units * nh_all * D; idx += NW * 64) {
-        const int us = idx / (nh_all * D);
-        const int r2 = idx - us * nh_all * D;
-        const int cc = r2 / D, d = r2 - cc * D;
-        const int u2 = ublk * shape.units + us;
-        // the last unit block of a geometry whose IU does not divide U has
-        // slots past the last unit: they own no output row
-        if (u2 >= a.U) continue;
-        const int hkv2 = u2 / a.HG, hg2 = u2 - hkv2 * a.HG;
-        if (16 * hg2 + cc >= a.G) continue;
-        float M = -INFINITY;
-        for (int p2 = 0; p2 < shape.P; ++p2) M = fmaxf(M, l_m[(us * shape.P + p2) * a.G16 + cc]);
-        float L = 0.f, A = 0.f;
-        if (M != -INFINITY) {
-          for (int p2 = 0; p2 < shape.P; ++p2) {
-            const int w2 = us * shape.P + p2;
-            const float mw = l_m[w2 * a.G16 + cc];
-            const float wt = (mw == -INFINITY) ? 0.f : fast_exp2(mw - M);
-            L += wt * l_l[w2 * a.G16 + cc];
-            A += wt * l_acc[(w2 * a.G16 + cc) * D + d];
+      // (a unit slot past the last unit owns no output row: nh = 0)
+      constexpr int DL = D / 64;
+      typedef float fDL __attribute__((ext_vector_type(DL)));
+      constexpr int PB = 4;      // states read together (one code path for P = 2, 4 and 8: two more cost registers)
+      const int w0 = wave - phase, w1 = w0 + shape.P - 1;
+      for (int cc = phase; cc < nh; cc += shape.P) {
+        float M = -INFINITY, L = 0.f;
+        fDL A = {};
+        for (int p0 = w0; p0 <= w1; p0 += PB) {
+          float mw[PB], lw[PB];
+          fDL x[PB];
+#pragma unroll
+          for (int p2 = 0; p2 < PB; ++p2) {
+            const int ws = min(p0 + p2, w1) * a.G16 + cc;
+            mw[p2] = l_m[ws];
+            lw[p2] = l_l[ws];
+            x[p2] = *(const fDL*)(l_acc + ws * D + DL * lane);
           }
+          float mb = M;
+#pragma unroll
+          for (int p2 = 0; p2 < PB; ++p2) {
+            if (p0 + p2 > w1) mw[p2] = -INFINITY;           // (the last state read again)
+            mb = fmaxf(mb, mw[p2]);
+          }
+          const float mref = mb == -INFINITY ? 0.f : mb;    // (a wave without a tile weighs 2^-inf = 0)
+          const float r = fast_exp2(M - mref);
+          L *= r;
+          A *= r;
+#pragma unroll
+          for (int p2 = 0; p2 < PB; ++p2) {
+            const float wt = fast_exp2(mw[p2] - mref);
+            L += wt * lw[p2];
+            A += wt * x[p2];
+          }
+          M = mb;
         }
-        const int hqo = hkv2 * a.G + 16 * hg2 + cc;
+        const int hqo = hkv * a.G + 16 * hg + cc;
         if (direct) {
-          char* op = a.out + b * a.o_sb + (int64_t)hqo * a.o_sh + d * (int)sizeof(uint16_t);
-          store_out(QT{}, op, A / (L == 0.f ? 1.f : L));
+          const float inv = 1.0f / (L == 0.f ? 1.f : L);
+          char* op = a.out + b * a.o_sb + (int64_t)hqo * a.o_sh + DL * lane * (int)sizeof(uint16_t);
+          if constexpr (DL == 1) {
+            store_out(QT{}, op, A[0] * inv);
+          } else {
+#pragma unroll
+            for (int e = 0; e < DL; e += 2) *(uint32_t*)(op + 2 * e) = pack2(QT{}, A[e] * inv, A[e + 1] * inv);
+          }
         } else {
-          const int64_t ps = ((int64_t)pslot_id * NW + us) * a.G16 + cc;
-          a.ws_acc[ps * D + d] = A;
-          if (d == 0) { a.ws_ml[ps * 2 + 0] = M; a.ws_ml[ps * 2 + 1] = L; }
+          const int64_t ps = ((int64_t)pslot_id * NW + uin) * a.G16 + cc;
+          *(fDL*)(a.ws_acc + ps * D + DL * lane) = A;
+          if (lane == 0) { a.ws_ml[ps * 2 + 0] = M; a.ws_ml[ps * 2 + 1] = L; }
         }
       }
     }
@@ -989,7 +1129,7 @@ __global__ __launch_bounds__(PW * 64) void decode_reduce(const DecodeArgs a) {
   const bool inr = row < a.B * a.Hq;
   // the plan's header and this row's prefix entries in one round trip
   // (loaded before any test of them, for rows past the end as well)
-  const int b = (inr ? row : 0) / a.Hq;
+  const int b = fdiv(inr ? row : 0, a.dHq);
   const int hq = (inr ? row : 0) - b * a.Hq;
   const int pb = a.ws_plan[kPlanHeader + b], pe = a.ws_plan[kPlanHeader + b + 1];
   const int W = a.ws_plan[kPlanW], G = a.ws_plan[kPlanG], pen = a.ws_plan[kPlanPen];
@@ -998,12 +1138,12 @@ __global__ __launch_bounds__(PW * 64) void decode_reduce(const DecodeArgs a) {
   // 2g) only if the range starts exactly at the group's start
   int nsplit = 1, gf = 0, s_first = 0, uin = 0, cc = 0;
   if (inr) {
-    const int nvt = (pe - pb) / a.UB;                // virtual tiles per unit block (0: empty sequence)
-    const int hkv = hq / a.G, gi = hq - hkv * a.G;
+    const int nvt = fdiv(pe - pb, a.dUB);            // virtual tiles per unit block (0: empty sequence)
+    const int hkv = fdiv(hq, a.dG), gi = hq - hkv * a.G;
     cc = gi & 15;
     const int unit = hkv * a.HG + (gi >> 4);
     const ItemShape shape = item_shape<NW>(a);
-    const int ublk = unit / shape.units;
+    const int ublk = fdiv(unit, a.dIU);
     uin = unit - ublk * shape.units;
     if (nvt == 0) {
       nsplit = 0;                                   // empty sequence: zeros
@@ -1012,9 +1152,10 @@ __global__ __launch_bounds__(PW * 64) void decode_reduce(const DecodeArgs a) {
       // after the first pen positions, held by groups gf .. (pieces); the
       // piece of gf is that group's first segment unless gf started before v0
       const int v0 = pb + ublk * nvt;
-      gf = sk_group(v0 + pen, W, G);
-      nsplit = sk_group(v0 + nvt - 1, W, G) - gf + 1;
-      s_first = sk_lo(gf, W, G) < v0 ? 1 : 0;
+      const SkSplit sk = sk_split(W, G);
+      gf = sk_group(sk, v0 + pen);
+      nsplit = sk_group(sk, v0 + nvt - 1) - gf + 1;
+      s_first = sk_lo(sk, gf) < v0 ? 1 : 0;
     }
   }
   const bool work = inr && nsplit != 1;

@@ -50,10 +50,19 @@ int launch_decode_typed(DecodeLaunch& L) {
   // time for 16-bit K/V and three for int8.  Equal lengths keep their shares
   // aligned to sequence boundaries whatever the charge.
   L.a.seg_pen = std::is_same<KV, I8>::value ? 3 : 2;
+  int lg = 0;
+  while ((2 << lg) <= NW / L.a.IU) ++lg;
+  L.a.lgP = lg;
+  L.a.dHG = make_fastdiv((uint32_t)L.a.HG);
+  L.a.dUB = make_fastdiv((uint32_t)L.a.UB);
+  L.a.dHq = make_fastdiv((uint32_t)L.a.Hq);
+  L.a.dG = make_fastdiv((uint32_t)L.a.G);
+  L.a.dIU = make_fastdiv((uint32_t)L.a.IU);
   const size_t lds = decode_lds_bytes(D, L.a.G16, L.a.B, NW);
   const int occ = kernel_occupancy((const void*)kmain, NW * 64, lds);
   if (occ <= 0) return fail(SIA_ERR_LAUNCH, "decode kernel does not fit on a CU (LDS %zu B)", lds);
   L.a.slots = device_info().cus * occ;
+  if (L.a.slots > 4095) L.a.slots = 4095;   // (the split's 24-bit arithmetic, sk_lo)
   // One length for the whole batch and a segment count ((sequence, unit
   // block) pairs) that is a multiple of the persistent grid: the split gives
   // every group whole segments, so decode_main writes every row itself
