@@ -26,7 +26,8 @@ from __future__ import annotations
 
 import torch
 
-from .decode import attention_flash_decode, attention_flash_decode_int8
+from .decode import (CONTIG, CONTIG_INT8, _common, _kv_len_tensor, _run_layer, attention_flash_decode,
+                     attention_flash_decode_int8)
 from .kv_cache import KVCache
 from .prefill import attention_flash_triton
 
@@ -80,12 +81,12 @@ def rope_decode_step_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     Returns ``(B, 1, Hq, D)``.  Graph safe.
     """
     q_rot = kv_cache.write_decode_rope(layer_idx, ctx.pos_index, q, k, v, cos, sin, interleaved=interleaved)
-    B = q.shape[0]
-    kc, vc, ks, vs = kv_cache._layer(layer_idx, B)
     qh = q_rot.transpose(1, 2)
-    if kv_cache.is_int8:
-        return attention_flash_decode_int8(qh, kc, vc, ks, vs, ctx.kv_len, sm_scale)
-    return attention_flash_decode(qh, kc, vc, ctx.kv_len, sm_scale)
+    scale = _common(qh, kv_cache.k_cache, sm_scale)
+    kl = _kv_len_tensor(ctx.kv_len, qh.device)
+    ks, vs = (kv_cache.k_scale, kv_cache.v_scale) if kv_cache.is_int8 else (None, None)
+    return _run_layer(CONTIG_INT8 if kv_cache.is_int8 else CONTIG, qh, kv_cache.k_cache, kv_cache.v_cache, ks, vs,
+                      layer_idx, None, kl, 0, scale)
 
 
 def decode_step_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_cache: KVCache, layer_idx: int,

@@ -101,13 +101,23 @@ def _run(kind: int, q: torch.Tensor, k, v, k_scale, v_scale, block_table, kv_len
     ops = _OPS
     if ops is None:
         ops = _OPS = _lib.gpu_ops()
-    tps = b = e = 0
-    if _opts_users:
-        tps = getattr(_tls, "tiles_per_split", 0)
-        ev = getattr(_tls, "main_events", None)
-        if ev is not None:
-            b, e = ev[0].cuda_event, ev[1].cuda_event
+    tps, b, e = _options() if _opts_users else (0, 0, 0)
     return ops.decode(kind, q, k, v, k_scale, v_scale, block_table, kv_len, page_size, sm_scale, tps, b, e)
+
+
+def _run_layer(kind: int, q: torch.Tensor, k, v, k_scale, v_scale, layer: int, block_table, kv_len, page_size: int,
+               sm_scale: float) -> torch.Tensor:
+    """One decode call over layer ``layer`` of a cache's whole ``(L, ...)`` pools (cut in C++, no views here)."""
+    tps, b, e = _options() if _opts_users else (0, 0, 0)
+    return _lib.gpu_ops().decode_layer(kind, q, k, v, k_scale, v_scale, layer, block_table, kv_len, page_size,
+                                       sm_scale, tps, b, e)
+
+
+def _options():
+    """(tiles per split, begin event, end event) of this thread's decode_options block."""
+    ev = getattr(_tls, "main_events", None)
+    b, e = (ev[0].cuda_event, ev[1].cuda_event) if ev is not None else (0, 0)
+    return getattr(_tls, "tiles_per_split", 0), b, e
 
 
 def _common(q: torch.Tensor, k: torch.Tensor, sm_scale):

@@ -163,10 +163,9 @@ class KVCache:
         sequence's position ``pos_index`` on the device, so no per-step table
         row copy is needed.
         """
-        B = k.shape[0]
-        kc, vc, ks, vs = self._layer(layer_idx, B)
-        return rope_kv_write(q, k, v, cos, sin, kc, vc, ks, vs, start_pos=_int32_positions(pos_index),
-                             interleaved=interleaved)
+        ks, vs = (self.k_scale, self.v_scale) if self.is_int8 else (None, None)
+        return _lib.gpu_ops().rope_kv_write_layer(q, k, v, cos, sin, self.k_cache, self.v_cache, ks, vs, layer_idx,
+                                                  None, _int32_positions(pos_index), 0, 0, bool(interleaved))
 
     def reset(self) -> None:
         """Logical reset between independent sequences (nothing to clear, as in the reference)."""

@@ -25,8 +25,9 @@ from __future__ import annotations
 
 import torch
 
-from .decode import paged_attention_flash_decode, paged_gqa_int8_flash_decode
-from .kv_cache import kv_write, rope_kv_write
+from . import _lib
+from .decode import PAGED, PAGED_INT8, _common, _run_layer
+from .kv_cache import kv_write
 
 
 class PagedKVCache:
@@ -123,21 +124,17 @@ class PagedKVCache:
         rotated by that row of the full ``cos``/``sin`` tables, so requests at
         different positions share one launch.
         """
-        B = k.shape[0]
-        kp, vp, ks, vs = self.layer(layer_idx)
-        return rope_kv_write(q, k, v, cos, sin, kp, vp, ks, vs, block_table=self.block_tables[:B],
-                             start_pos=self.seq_lens[:B], start_offset=-1, page_size=self.block_size,
-                             interleaved=interleaved)
+        ks, vs = (self.k_scale_pool, self.v_scale_pool) if self.is_int8 else (None, None)
+        return _lib.gpu_ops().rope_kv_write_layer(q, k, v, cos, sin, self.k_pool, self.v_pool, ks, vs, layer_idx,
+                                                  self.block_tables, self.seq_lens, -1, self.block_size,
+                                                  bool(interleaved))
 
     def decode_attention(self, layer_idx: int, q: torch.Tensor, sm_scale: float | None = None) -> torch.Tensor:
         """Decode attention of ``q (B, Hq, 1, D)`` over each request's ``seq_lens[b]`` cached tokens."""
-        B = q.shape[0]
-        kp, vp, ks, vs = self.layer(layer_idx)
-        if self.is_int8:
-            return paged_gqa_int8_flash_decode(q, kp, vp, ks, vs, self.block_tables[:B], self.seq_lens[:B],
-                                               self.block_size, sm_scale)
-        return paged_attention_flash_decode(q, kp, vp, self.block_tables[:B], self.seq_lens[:B],
-                                            self.block_size, sm_scale)
+        scale = _common(q, self.k_pool, sm_scale)
+        ks, vs = (self.k_scale_pool, self.v_scale_pool) if self.is_int8 else (None, None)
+        return _run_layer(PAGED_INT8 if self.is_int8 else PAGED, q, self.k_pool, self.v_pool, ks, vs, layer_idx,
+                          self.block_tables, self.seq_lens, self.block_size, scale)
 
     def __repr__(self):
         gb = 2 * self.k_pool.numel() * self.k_pool.element_size() / 1e9

@@ -88,6 +88,63 @@ struct OptDesc {
   const sia_tensor* ptr() const { return set ? &d : nullptr; }
 };
 
+// A descriptor limited to the first n entries of its first dimension (t[:n]).
+sia_tensor first_rows(sia_tensor d, int64_t n) {
+  if (d.ndim > 0 && n < d.shape[0]) d.shape[0] = n;
+  return d;
+}
+
+// pool[layer] of a cache's (L, ...) pools, as a descriptor.  Cutting the views
+// in Python instead, by layer and by batch and once per launch, kept the host
+// behind the GPU: a decode step of one int8 sequence of 1000 tokens took 25.4
+// us per call, 17.3 this way; a paged one of 8 bf16 requests 22.2 and 19.5.
+sia_tensor layer_desc(const Tensor& pool, int64_t layer, const at::Device& dev, const char* name) {
+  sia_tensor d = desc(pool, dev, name);
+  if (d.ndim < 1) throw py::value_error(std::string(name) + " must have a layer dimension");
+  if (layer < 0) layer += d.shape[0];
+  if (layer < 0 || layer >= d.shape[0])
+    throw py::index_error(std::string("layer index out of range for ") + name + " of " + std::to_string(d.shape[0]) +
+                          " layers");
+  d.data = (char*)d.data + layer * d.stride[0] * (int64_t)pool.element_size();
+  --d.ndim;
+  for (int i = 0; i < d.ndim; ++i) {
+    d.shape[i] = d.shape[i + 1];
+    d.stride[i] = d.stride[i + 1];
+  }
+  return d;
+}
+
+// One layer of a KV cache: contiguous pools (L, B', H, S, D) cut to the first
+// B sequences, or paged pools (L, N, H, P, D) with the block table's first B
+// rows.
+struct LayerDescs {
+  sia_tensor k, v, ks, vs, bt;
+  bool has_scales, has_bt;
+  LayerDescs(const Tensor& kp, const Tensor& vp, const OptT& ksp, const OptT& vsp, const OptT& block_table,
+             int64_t layer, int64_t B, const at::Device& dev)
+      : has_scales(ksp.has_value() && vsp.has_value()), has_bt(block_table.has_value()) {
+    k = layer_desc(kp, layer, dev, "k cache");
+    v = layer_desc(vp, layer, dev, "v cache");
+    if (has_scales) {
+      ks = layer_desc(*ksp, layer, dev, "k scales");
+      vs = layer_desc(*vsp, layer, dev, "v scales");
+    }
+    if (has_bt) {
+      bt = first_rows(desc(*block_table, dev, "block_table"), B);
+    } else {
+      k = first_rows(k, B);
+      v = first_rows(v, B);
+      if (has_scales) {
+        ks = first_rows(ks, B);
+        vs = first_rows(vs, B);
+      }
+    }
+  }
+  const sia_tensor* ksp() const { return has_scales ? &ks : nullptr; }
+  const sia_tensor* vsp() const { return has_scales ? &vs : nullptr; }
+  const sia_tensor* btp() const { return has_bt ? &bt : nullptr; }
+};
+
 at::Device gpu_of(const Tensor& t, const char* name) {
   if (!t.is_cuda())
     throw py::value_error(std::string("the attention kernels run on the GPU: ") + name +
@@ -118,6 +175,11 @@ size_t decode_ws_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int dev) {
 
 enum DecodeKind { kContig = 0, kContigInt8 = 1, kGqaInt8 = 2, kPaged = 3, kPagedInt8 = 4 };
 
+Tensor decode_call(int64_t kind, const Tensor& q, const sia_tensor& dk, const sia_tensor& dv, const sia_tensor* dks,
+                   const sia_tensor* dvs, const sia_tensor* dbt, const sia_tensor& dl, int64_t page_size,
+                   double sm_scale, int64_t tiles_per_split, int64_t begin_event, int64_t end_event,
+                   const at::Device& dev);
+
 // One decode call (q (B, Hq, 1, D)) -> out (B, 1, Hq, D) in q's dtype.
 Tensor decode(int64_t kind, const Tensor& q, const Tensor& k, const Tensor& v, const OptT& k_scale,
               const OptT& v_scale, const OptT& block_table, const Tensor& kv_len, int64_t page_size, double sm_scale,
@@ -126,13 +188,42 @@ Tensor decode(int64_t kind, const Tensor& q, const Tensor& k, const Tensor& v, c
   const c10::DeviceGuard guard(dev);
   if (q.dim() != 4) throw py::value_error("q must be (B, Hq, 1, D)");
   if (k.dim() != 4) throw py::value_error("k must have 4 dims");
-  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), Hkv = k.size(1);
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3);
   // an empty batch has nothing to compute (the reference's launch over a
   // grid of B * Hq programs does nothing either)
   if (B == 0) return at::empty({0, 1, Hq, D}, q.options());
-  const sia_tensor dq = desc(q, dev, "q"), dk = desc(k, dev, "k"), dv = desc(v, dev, "v");
+  const sia_tensor dk = desc(k, dev, "k"), dv = desc(v, dev, "v");
   const sia_tensor dl = desc(kv_len, dev, "kv_len");
   const OptDesc dks(k_scale, dev, "k_scale"), dvs(v_scale, dev, "v_scale"), dbt(block_table, dev, "block_table");
+  return decode_call(kind, q, dk, dv, dks.ptr(), dvs.ptr(), dbt.ptr(), dl, page_size, sm_scale, tiles_per_split,
+                     begin_event, end_event, dev);
+}
+
+// The same over layer `layer` of a cache's whole pools; kv_len is cut to the
+// first B entries with a block table (one length per request there).
+Tensor decode_layer(int64_t kind, const Tensor& q, const Tensor& k_pool, const Tensor& v_pool, const OptT& k_scales,
+                    const OptT& v_scales, int64_t layer, const OptT& block_table, const Tensor& kv_len,
+                    int64_t page_size, double sm_scale, int64_t tiles_per_split, int64_t begin_event,
+                    int64_t end_event) {
+  const at::Device dev = gpu_of(q, "q");
+  const c10::DeviceGuard guard(dev);
+  if (q.dim() != 4) throw py::value_error("q must be (B, Hq, 1, D)");
+  if (k_pool.dim() != 5) throw py::value_error("the cache's k must have 5 dims");
+  const int64_t B = q.size(0);
+  if (B == 0) return at::empty({0, 1, q.size(1), q.size(3)}, q.options());
+  const LayerDescs c(k_pool, v_pool, k_scales, v_scales, block_table, layer, B, dev);
+  sia_tensor dl = desc(kv_len, dev, "kv_len");
+  if (c.has_bt) dl = first_rows(dl, B);
+  return decode_call(kind, q, c.k, c.v, c.ksp(), c.vsp(), c.btp(), dl, page_size, sm_scale, tiles_per_split,
+                     begin_event, end_event, dev);
+}
+
+Tensor decode_call(int64_t kind, const Tensor& q, const sia_tensor& dk, const sia_tensor& dv, const sia_tensor* dks,
+                   const sia_tensor* dvs, const sia_tensor* dbt, const sia_tensor& dl, int64_t page_size,
+                   double sm_scale, int64_t tiles_per_split, int64_t begin_event, int64_t end_event,
+                   const at::Device& dev) {
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), Hkv = dk.shape[1];
+  const sia_tensor dq = desc(q, dev, "q");
   Tensor out = at::empty({B, 1, Hq, D}, q.options());
   const sia_tensor dout = desc(out, dev, "out");
   const size_t ws_bytes = decode_ws_bytes(B, Hq, Hkv, D, dev.index());
@@ -151,20 +242,18 @@ Tensor decode(int64_t kind, const Tensor& q, const Tensor& k, const Tensor& v, c
       rc = sia_attention_flash_decode(&dq, &dk, &dv, &dl, sc, &dout, ws.data_ptr(), ws_bytes, po, s);
       break;
     case kContigInt8:
-      rc = sia_attention_flash_decode_int8(&dq, &dk, &dv, dks.ptr(), dvs.ptr(), &dl, sc, &dout, ws.data_ptr(),
-                                           ws_bytes, po, s);
+      rc = sia_attention_flash_decode_int8(&dq, &dk, &dv, dks, dvs, &dl, sc, &dout, ws.data_ptr(), ws_bytes, po, s);
       break;
     case kGqaInt8:
-      rc = sia_gqa_int8_flash_decode(&dq, &dk, &dv, dks.ptr(), dvs.ptr(), &dl, sc, &dout, ws.data_ptr(), ws_bytes,
-                                     po, s);
+      rc = sia_gqa_int8_flash_decode(&dq, &dk, &dv, dks, dvs, &dl, sc, &dout, ws.data_ptr(), ws_bytes, po, s);
       break;
     case kPaged:
-      rc = sia_paged_attention_flash_decode(&dq, &dk, &dv, dbt.ptr(), &dl, (int32_t)page_size, sc, &dout,
-                                            ws.data_ptr(), ws_bytes, po, s);
+      rc = sia_paged_attention_flash_decode(&dq, &dk, &dv, dbt, &dl, (int32_t)page_size, sc, &dout, ws.data_ptr(),
+                                            ws_bytes, po, s);
       break;
     case kPagedInt8:
-      rc = sia_paged_gqa_int8_flash_decode(&dq, &dk, &dv, dks.ptr(), dvs.ptr(), dbt.ptr(), &dl, (int32_t)page_size,
-                                           sc, &dout, ws.data_ptr(), ws_bytes, po, s);
+      rc = sia_paged_gqa_int8_flash_decode(&dq, &dk, &dv, dks, dvs, dbt, &dl, (int32_t)page_size, sc, &dout,
+                                           ws.data_ptr(), ws_bytes, po, s);
       break;
     default:
       throw py::value_error("unknown decode kind");
@@ -282,6 +371,29 @@ OptT rope_kv_write(const OptT& q, const Tensor& k, const OptT& v, const Tensor& 
   return qo;
 }
 
+// rope_kv_write into layer `layer` of a cache's whole pools, the decode step's
+// write: position start_offset + start_pos[b], which with a block table is cut
+// to the first B entries (one length per request there).
+OptT rope_kv_write_layer(const OptT& q, const Tensor& k, const OptT& v, const Tensor& cos, const Tensor& sin,
+                         const Tensor& k_pool, const Tensor& v_pool, const OptT& k_scales, const OptT& v_scales,
+                         int64_t layer, const OptT& block_table, const Tensor& start_pos, int64_t start_offset,
+                         int64_t page_size, bool interleaved) {
+  const at::Device dev = gpu_of(k, "k");
+  const c10::DeviceGuard guard(dev);
+  OptT qo;
+  if (q.has_value()) qo = at::empty(q->sizes(), q->options());
+  if (k.dim() < 1) throw py::value_error("k must be (B, T, H, D)");
+  if (k.numel() == 0 && k.dim() == 4 && (!q.has_value() || q->numel() == 0)) return qo;   // no tokens
+  const LayerDescs c(k_pool, v_pool, k_scales, v_scales, block_table, layer, k.size(0), dev);
+  const sia_tensor dk = desc(k, dev, "k"), dc = desc(cos, dev, "cos"), dsn = desc(sin, dev, "sin");
+  const OptDesc dq(q, dev, "q"), dv(v, dev, "v"), dqo(qo, dev, "q_out");
+  sia_tensor dsp = desc(start_pos, dev, "start_pos");
+  if (c.has_bt) dsp = first_rows(dsp, k.size(0));
+  check(sia_rope_kv_write(dq.ptr(), &dk, dv.ptr(), &dc, &dsn, interleaved ? 1 : 0, dqo.ptr(), &c.k, &c.v, c.ksp(),
+                          c.vsp(), c.btp(), &dsp, (int32_t)start_offset, (int32_t)page_size, stream_of(dev)));
+  return qo;
+}
+
 // A (B, T, H, D) view whose B*T rows sit one stride apart (head_dim
 // unit-stride, heads D apart), as sia_rope_qk reads it; other views are
 // copied first (kernels/rope_kernel.py:216-235 does the same).
@@ -329,10 +441,12 @@ PYBIND11_MODULE(_sia_ops, m) {
     return n;
   });
   m.def("decode", &decode);
+  m.def("decode_layer", &decode_layer);
   m.def("prefill", &prefill);
   m.def("prefill_rope", &prefill_rope);
   m.def("quantize_kv_int8", &quantize_kv_int8);
   m.def("kv_write", &kv_write);
   m.def("rope_kv_write", &rope_kv_write);
+  m.def("rope_kv_write_layer", &rope_kv_write_layer);
   m.def("rope_qk", &rope_qk);
 }
