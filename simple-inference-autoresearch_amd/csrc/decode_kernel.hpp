@@ -48,6 +48,14 @@ constexpr int kTile = 16;          // tokens per MFMA tile
 // per sequence (B+1 ints) follows.
 constexpr int kPlanW = 0, kPlanG = 1, kPlanUB = 2, kPlanPen = 3, kPlanHeader = 4;
 constexpr int kMinWaveTiles = 2;   // least work per work-group: this many tiles per wave of a unit
+// int8 K/V at head_dim 64 fits two groups per CU; the second one per CU joins
+// from this many tiles per wave on.  Below, its pieces mostly cost more in
+// starts and merging than they hide: one group per CU / two, 32/8 heads, fp16
+// scales, us per call: 2 tiles (8 sequences of 750-3000 tokens) 15.4 / 18.9,
+// 3.9 (4 x 8000) 16.5 / 18.2, 4.9 (16 x 1000-4000) 22.0 / 22.5 but (32 x
+// 500-2000) 27.5 / 25.1, 5.2 (64 x 250-1000) 27.0 / 25.5, 8 (256 log-normal
+// lengths up to 2000) 48.2 / 43.2.
+constexpr int kTwoGroupTiles = 5;
 // The running max is only raised when a score exceeds it by more than this
 // (log2 units), so p = 2^(s - m) <= 2^8: well inside f16/bf16 range, and the
 // rescale of (l, acc) almost never runs after the first tile.
@@ -74,6 +82,7 @@ struct DecodeArgs {
   int32_t tps_force;
   int32_t seg_pen;                                   // virtual tiles charged to each segment start (the split)
   int32_t slots;                                     // persistent work-groups of decode_main
+  int32_t cus;                                       // CUs
   int32_t scale_vec;                                 // scale rows allow one vector load per lane
   int32_t direct_only;                               // no decode_reduce follows: empty calls write zeros here
   // 32-bit copies of the per-tile strides (bytes): page strides (0 when
@@ -245,8 +254,22 @@ __device__ __forceinline__ int sk_group(const SkSplit& s, int x) {
 
 // -------------------------------------------------------------- tile data
 
+// int8 scales of a lane's 4 tokens.  fp16 scales stay as loaded until they are
+// used (two packed words from a scale vector, else one word each): converted
+// at the load, they took 4 registers per tile more and every round of the
+// tile loop waited for its last load.
+template <class ST, bool SV>
+struct Scales { float f[4]; };
+template <bool SV>
+struct Scales<F16, SV> { uint32_t w[SV ? 2 : 4]; };
+template <class ST, bool SV>
+__device__ __forceinline__ float scale_of(const Scales<ST, SV>& s, int i) {
+  if constexpr (std::is_same<ST, F32>::value) return s.f[i];
+  else return SV ? ((i & 1) ? hi_f32(F16{}, s.w[i >> 1]) : lo_f32(F16{}, s.w[i >> 1])) : lo_f32(F16{}, s.w[i]);
+}
+
 // One 16-token tile's operands as held by one lane.
-template <int D, class KV, class ST>
+template <int D, class KV, class ST, bool SV>
 struct Tile {
   // K bytes per lane, token lane16: 16 bytes per MFMA k-step j, at bytes
   // [64 j + 16 grp, +16) of the row (elements [32 j + 8 grp, +8) for 16-bit
@@ -265,7 +288,7 @@ struct Tile {
   static constexpr bool kVSplit = !kInt8 && VB > 16;
   Raw<KB> k;
   Raw<VB> v[4];                                      // tokens 4*grp + i
-  float ks[4], vs[4];                                // int8 scales of tokens 4*grp + i
+  Scales<ST, SV> ks, vs;                             // int8 scales of tokens 4*grp + i
 };
 
 // This lane's byte offsets inside one tile (constant): K of token lane16
@@ -315,10 +338,11 @@ __device__ __forceinline__ float load_scale(const char* p) {
   if constexpr (std::is_same<ST, F32>::value) return *(const float*)p;
   else return (float)*(const _Float16*)p;
 }
+// (the bits: fp32, or fp16 in the low half)
 template <class ST>
-__device__ __forceinline__ float load_scale(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  if constexpr (std::is_same<ST, F32>::value) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, kLoadNT));
-  else return (float)__builtin_bit_cast(_Float16, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, kLoadNT));
+__device__ __forceinline__ uint32_t load_scale(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  if constexpr (std::is_same<ST, F32>::value) return __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, kLoadNT);
+  else return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, kLoadNT);
 }
 
 // Load this lane's operands of one tile.  FULL: all 16 tokens exist, so no
@@ -329,8 +353,8 @@ __device__ __forceinline__ float load_scale(__amdgpu_buffer_rsrc_t rs, uint32_t 
 // (a branch there makes the compiler wait for the next tile's loads as well).
 template <int D, class KV, class ST, bool FULL, bool SV>
 __device__ __forceinline__ void load_tile(const DecodeArgs& a, const TilePtr& t, const LaneOff& o, int valid,
-                                          Tile<D, KV, ST>& c, int lane16, int grp) {
-  using C = Tile<D, KV, ST>;
+                                          Tile<D, KV, ST, SV>& c, int lane16, int grp) {
+  using C = Tile<D, KV, ST, SV>;
   const __amdgpu_buffer_rsrc_t rk = tile_rsrc(t.k), rv = tile_rsrc(t.v);
   if (FULL || lane16 < valid) load_raw_buf<C::KB, C::KSTRIDE>(c.k, rk, o.k);
   else zero_raw<C::KB>(c.k);
@@ -345,29 +369,37 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, const TilePtr& t,
       const u32x4 k4 = __builtin_amdgcn_raw_buffer_load_b128(rks, o.ks, 0, kLoadNT);
       const u32x4 v4 = __builtin_amdgcn_raw_buffer_load_b128(rvs, o.vs, 0, kLoadNT);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) { c.ks[i] = __uint_as_float(k4[i]); c.vs[i] = __uint_as_float(v4[i]); }
+      for (int i = 0; i < 4; ++i) { c.ks.f[i] = __uint_as_float(k4[i]); c.vs.f[i] = __uint_as_float(v4[i]); }
     } else if constexpr (FULL && SV) {   // fp16 scale rows: the 4 scales in one 8-byte load
       const u32x2 k2 = __builtin_amdgcn_raw_buffer_load_b64(rks, o.ks, 0, kLoadNT);
       const u32x2 v2 = __builtin_amdgcn_raw_buffer_load_b64(rvs, o.vs, 0, kLoadNT);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        c.ks[i] = (float)__builtin_bit_cast(_Float16, (unsigned short)(k2[i >> 1] >> (16 * (i & 1))));
-        c.vs[i] = (float)__builtin_bit_cast(_Float16, (unsigned short)(v2[i >> 1] >> (16 * (i & 1))));
-      }
+      for (int i = 0; i < 2; ++i) { c.ks.w[i] = k2[i]; c.vs.w[i] = v2[i]; }
     } else {
+      uint32_t k1[4], v1[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bool ok = FULL || 4 * grp + i < valid;
-        c.ks[i] = ok ? load_scale<ST>(rks, o.ks + i * a.ks_tok) : 0.0f;
-        c.vs[i] = ok ? load_scale<ST>(rvs, o.vs + i * a.vs_tok) : 0.0f;
+        k1[i] = ok ? load_scale<ST>(rks, o.ks + i * a.ks_tok) : 0u;
+        v1[i] = ok ? load_scale<ST>(rvs, o.vs + i * a.vs_tok) : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (std::is_same<ST, F32>::value) {
+          c.ks.f[i] = __uint_as_float(k1[i]); c.vs.f[i] = __uint_as_float(v1[i]);
+        } else if constexpr (!SV) {
+          c.ks.w[i] = k1[i]; c.vs.w[i] = v1[i];
+        } else if (i & 1) {
+          c.ks.w[i >> 1] = k1[i - 1] | k1[i] << 16; c.vs.w[i >> 1] = v1[i - 1] | v1[i] << 16;
+        }
       }
     }
   }
 }
 
 // K operand (A of S^T = K Q^T) for k-step j: 8 elements as 4 words.
-template <int D, class KV, class ST>
-__device__ __forceinline__ u32x4 k_operand(const Tile<D, KV, ST>& c, int j) {
+template <int D, class KV, class ST, bool SV>
+__device__ __forceinline__ u32x4 k_operand(const Tile<D, KV, ST, SV>& c, int j) {
   u32x4 r;
   if constexpr (std::is_same<KV, I8>::value) {
     const uint32_t w0 = c.k.w[2 * j] ^ 0x80808080u;
@@ -387,8 +419,8 @@ __device__ __forceinline__ u32x4 k_operand(const Tile<D, KV, ST>& c, int j) {
 
 // V^T operand (A of O^T += V^T P^T, 16x16x16) for d-tile e: element e of the
 // lane's D/16-wide slice for tokens (4g, 4g+1) and (4g+2, 4g+3).
-template <int D, class KV, class ST>
-__device__ __forceinline__ u32x2 v_operand(const Tile<D, KV, ST>& c, int e) {
+template <int D, class KV, class ST, bool SV>
+__device__ __forceinline__ u32x2 v_operand(const Tile<D, KV, ST, SV>& c, int e) {
   u32x2 r;
   if constexpr (std::is_same<KV, I8>::value) {
     r[0] = i8gather_to_f16x2(c.v[0].w[e >> 2], c.v[1].w[e >> 2], e & 3);
@@ -422,8 +454,8 @@ struct WaveState {
   f32x4 acc[D / 16];
 };
 
-template <int D, class KV, class QT, class ST, bool FULL>
-__device__ __forceinline__ void compute_tile(const Tile<D, KV, ST>& c, const u32x4* qop, const u32x4* qop_lo,
+template <int D, class KV, class QT, class ST, bool FULL, bool SV>
+__device__ __forceinline__ void compute_tile(const Tile<D, KV, ST, SV>& c, const u32x4* qop, const u32x4* qop_lo,
                                              float qmul, int tile, int ntok, int grp, WaveState<D>& st) {
   using MT = typename MmaOf<KV>::T;
   constexpr int KSTEPS = D / 32;
@@ -451,13 +483,13 @@ __device__ __forceinline__ void compute_tile(const Tile<D, KV, ST>& c, const u32
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = __mul24(shi[i], 254) + smid[i];          // |t| < 2^30: exact
-      s[i] = __builtin_fmaf((float)t, 254.0f, (float)slo[i]) * (qmul * c.ks[i]);
+      s[i] = __builtin_fmaf((float)t, 254.0f, (float)slo[i]) * (qmul * scale_of(c.ks, i));
     }
   } else {
     f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < KSTEPS; ++j) {
-      const u32x4 ka = k_operand<D, KV, ST>(c, j);
+      const u32x4 ka = k_operand(c, j);
       sacc = mfma16x16x32(MT{}, ka, qop[j], sacc);
       if constexpr (QSplit<KV, QT>::value) sacc = mfma16x16x32(MT{}, ka, qop_lo[j], sacc);
     }
@@ -486,7 +518,8 @@ __device__ __forceinline__ void compute_tile(const Tile<D, KV, ST>& c, const u32
   u32x2 pop, pop_lo;
   if constexpr (kInt8) {
     // P' = p * s_v * 2^(4-sexp) stays < 2^12: p <= 2^kLazyMax and 2^sexp bounds every s_v seen.
-    const float lv = fmaxf(fmaxf(c.vs[0], c.vs[1]), fmaxf(c.vs[2], c.vs[3]));
+    const float vs0 = scale_of(c.vs, 0), vs1 = scale_of(c.vs, 1), vs2 = scale_of(c.vs, 2), vs3 = scale_of(c.vs, 3);
+    const float lv = fmaxf(fmaxf(vs0, vs1), fmaxf(vs2, vs3));
     if (__any(lv > ldexpf(1.0f, st.sexp))) {
       const float vmax = wave_max_xor16_32(lv);
       const int e_new = max(st.sexp, __builtin_amdgcn_frexp_expf(vmax));
@@ -495,8 +528,8 @@ __device__ __forceinline__ void compute_tile(const Tile<D, KV, ST>& c, const u32
       rescale = true;
     }
     const float rho = ldexpf(16.0f, -st.sexp);
-    pop[0] = pack2(F16{}, p[0] * (c.vs[0] * rho), p[1] * (c.vs[1] * rho));
-    pop[1] = pack2(F16{}, p[2] * (c.vs[2] * rho), p[3] * (c.vs[3] * rho));
+    pop[0] = pack2(F16{}, p[0] * (vs0 * rho), p[1] * (vs1 * rho));
+    pop[1] = pack2(F16{}, p[2] * (vs2 * rho), p[3] * (vs3 * rho));
   } else {
     pop[0] = pack2(MT{}, p[0], p[1]);
     pop[1] = pack2(MT{}, p[2], p[3]);
@@ -514,7 +547,7 @@ __device__ __forceinline__ void compute_tile(const Tile<D, KV, ST>& c, const u32
   st.l += (p[0] + p[1]) + (p[2] + p[3]);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const u32x2 va = v_operand<D, KV, ST>(c, e);
+    const u32x2 va = v_operand(c, e);
     st.acc[e] = mfma16x16x16(MT{}, va, pop, st.acc[e]);
     if constexpr (kPSplit) st.acc[e] = mfma16x16x16(MT{}, va, pop_lo, st.acc[e]);
   }
@@ -630,17 +663,17 @@ __device__ __forceinline__ float prep_q(const DecodeArgs& a, const QRaw<D>& raw,
 // 4 g + i loaded as element e of its V share (see Tile).
 template <int D, class KV>
 __device__ __forceinline__ int out_d(int g, int i, int e) {
-  if constexpr (Tile<D, KV, F32>::kVSplit) return 128 * (e >> 3) + 32 * g + 8 * i + (e & 7);
+  if constexpr (Tile<D, KV, F32, false>::kVSplit) return 128 * (e >> 3) + 32 * g + 8 * i + (e & 7);
   else return g * (D / 4) + i * (D / 16) + e;
 }
 
 // Waves per SIMD each instantiation is compiled for (its VGPR budget).  A
 // work-group is NW = 8 waves, so below 4 waves per SIMD a CU holds one group.
-// int8 at D = 64 gets 256 registers too: its int8 query split, scales and
-// conversions do not fit 128 without scratch spills.
-template <int D, class KV>
+// int8 at D = 64 with scattered scales gets 256 registers too: it does not fit
+// 128 without scratch spills (with scale vectors it takes 126).
+template <int D, class KV, bool SV>
 struct DecodeWaves {
-  static constexpr int value = D <= 64 && !std::is_same<KV, I8>::value ? 4 : (D <= 128 ? 2 : 1);
+  static constexpr int value = D <= 64 && (!std::is_same<KV, I8>::value || SV) ? 4 : (D <= 128 ? 2 : 1);
 };
 
 // Geometry of one item inside a work-group of NW waves (all uniform): it
@@ -677,7 +710,7 @@ __device__ __forceinline__ int aligned_groups(const DecodeArgs& a, int nt, int G
 }
 
 template <int D, class KV, class QT, class ST, int NW, bool SV>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DecodeWaves<D, KV>::value)))
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DecodeWaves<D, KV, SV>::value)))
 void decode_main(const DecodeArgs a) {
   constexpr int E = D / 16;
   constexpr int KSTEPS = D / 32;
@@ -705,6 +738,11 @@ void decode_main(const DecodeArgs a) {
   // segments on one group took ~50 us)
   G = min(G, max(a.B * a.UB, (W + kMinWaveTiles * shape.P - 1) / (kMinWaveTiles * shape.P)));
   G = min(G, max(1, a.max_items / 2));                      // two partial slots per group
+  // (one segment per CU, all of one length: whole segments, nothing to merge,
+  // 20.3 against 22.9 us at 64 x 1024 tokens)
+  if (std::is_same<KV, I8>::value && a.tps_force <= 0 && G > a.cus &&
+      (W < kTwoGroupTiles * shape.P * G || (pen == 0 && a.B * a.UB == a.cus)))
+    G = min(G, max(a.cus, a.B * a.UB));
   const int nt0 = (tok0 + kTile - 1) / kTile;               // (one shared length)
   if (!a.kv_per_seq && a.tps_force <= 0) G = aligned_groups(a, nt0, G, shape.P, KV::bytes * D);
   if (blockIdx.x == 0) {
@@ -739,7 +777,7 @@ void decode_main(const DecodeArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int lane16 = lane & 15, grp = lane >> 4;
-  using TileT = Tile<D, KV, ST>;
+  using TileT = Tile<D, KV, ST, SV>;
   LaneOff lo;
   lo.k = lane16 * a.k_tok + (uint32_t)(grp * 16);
 #pragma unroll
@@ -801,9 +839,9 @@ void decode_main(const DecodeArgs a) {
   // The next segment's query row and first page id are loaded while the
   // current one streams (seg_next: the start of the segment they belong
   // to), so that a segment change waits for its first tile only.
-  // (Not where its registers do not fit: 16-bit K/V at head_dim 64 in 128
-  // registers, int8 with scattered scales.)
-  constexpr bool kNext = TileT::kInt8 ? SV : D > 64;
+  // (Not where its registers do not fit: head_dim 64, two groups per CU in 128
+  // registers, and int8 with scattered scales.)
+  constexpr bool kNext = D > 64 && (!TileT::kInt8 || SV);
   QRaw<D> q_next;
   int pg_next = 0, seg_next = -1;
   bool first_seg = true;
@@ -853,7 +891,7 @@ void decode_main(const DecodeArgs a) {
       // already in flight), unless the previous segment loaded them already.
       QRaw<D> qraw;
       int pg0;
-      constexpr bool kPartFirst = D > 64 || TileT::kInt8;   // (see below)
+      constexpr bool kPartFirst = D > 64;   // (see below)
       int pgl = kPartFirst && nt > nfull ? page_id(nfull) : 0;
       if (kNext && x == seg_next) {
         qraw = q_next;
@@ -909,19 +947,24 @@ void decode_main(const DecodeArgs a) {
       // computed first (its order is free), while the first full tile is in
       // flight: behind the full tiles it was one more dependent round trip of
       // the wave that every other wave of the unit waited for, 2 us at one
-      // sequence of 1000 tokens.  (16-bit K/V at head_dim 64 has no registers
-      // for it in its 128, spills cost 4-17%, and takes it last.)
+      // sequence of 1000 tokens.  head_dim 64 takes it last: its 128
+      // registers (two groups per CU) hold no third tile.  (int8 with fp16 scales
+      // took 153 with one, so one group per CU: 256 log-normal lengths up to
+      // 2000, 32/8 heads, 50.0 us against 43.8, 64 sequences of 500-2000
+      // tokens, 16/16 heads, 51.1 against 43.5.  At one sequence of 1000 tokens
+      // it costs 0.6 us.)
+      auto load_part = [&](TileT& last) {
+        load_tile<D, KV, ST, false, SV>(a, tile_ptr(t_first + nfull * P, pgl), lo,
+                                           ntok - (t_first + nfull * P) * kTile, last, lane16, grp);
+      };
+      auto compute_part = [&](const TileT& last) {
+        compute_tile<D, KV, QT, ST, false>(last, qop, qop_lo, qmul, t_first + nfull * P, ntok, grp, st);
+      };
       const bool part = nt > nfull;
-      TileT last;
-      auto load_part = [&]() {
-        if (part)
-          load_tile<D, KV, ST, false, false>(a, tile_ptr(t_first + nfull * P, pgl), lo,
-                                             ntok - (t_first + nfull * P) * kTile, last, lane16, grp);
-      };
-      auto compute_part = [&]() {
-        if (part) compute_tile<D, KV, QT, ST, false>(last, qop, qop_lo, qmul, t_first + nfull * P, ntok, grp, st);
-      };
-      if constexpr (kPartFirst) load_part();
+      std::conditional_t<kPartFirst, TileT, int> first;     // (the partial tile, where it is taken first)
+      if constexpr (kPartFirst) {
+        if (part) load_part(first);
+      }
       // Full tiles, double-buffered.  The steady-state loop always issues the
       // next tiles' loads, and fetches the page ids of the tiles two ahead
       // with one vector load (lanes 0 and 1; indices clamped to the wave's
@@ -943,7 +986,9 @@ void decode_main(const DecodeArgs a) {
         prefetch_next();
         // the query's conversion overlaps the first tile's flight
         qmul = prep_q<D, KV, QT>(a, qraw, qop, qop_lo);
-        if constexpr (kPartFirst) compute_part();
+        if constexpr (kPartFirst) {
+          if (part) compute_part(first);
+        }
         int k = 0;
         for (; k + 2 < nfull; k += 2) {
           // With 8 waves, waves w and w^4 share a SIMD, where the older one
@@ -982,11 +1027,16 @@ void decode_main(const DecodeArgs a) {
       } else {
         prefetch_next();
         qmul = prep_q<D, KV, QT>(a, qraw, qop, qop_lo);
-        if constexpr (kPartFirst) compute_part();
+        if constexpr (kPartFirst) {
+          if (part) compute_part(first);
+        }
       }
       if constexpr (!kPartFirst) {
-        load_part();
-        compute_part();
+        if (part) {
+          TileT last;
+          load_part(last);
+          compute_part(last);
+        }
       }
     }
 

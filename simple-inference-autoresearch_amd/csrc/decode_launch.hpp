@@ -61,8 +61,15 @@ int launch_decode_typed(DecodeLaunch& L) {
   const size_t lds = decode_lds_bytes(D, L.a.G16, L.a.B, NW);
   const int occ = kernel_occupancy((const void*)kmain, NW * 64, lds);
   if (occ <= 0) return fail(SIA_ERR_LAUNCH, "decode kernel does not fit on a CU (LDS %zu B)", lds);
-  L.a.slots = device_info().cus * occ;
+  L.a.cus = device_info().cus;
+  L.a.slots = L.a.cus * occ;
   if (L.a.slots > 4095) L.a.slots = 4095;   // (the split's 24-bit arithmetic, sk_lo)
+  // int8 K/V at one shared length: one group per CU, also where two fit
+  // (head_dim 64).  No ragged starts for the second to hide (see
+  // kTwoGroupTiles), and a grid twice as large costs: fp16 scales, 32/8 heads,
+  // 32 x 512 tokens 9.7 against 11.6 us, 256 x 1000 56.5 against 58.8.
+  if (std::is_same<KV, I8>::value && !L.a.kv_per_seq && L.a.tps_force == 0 && L.a.slots > L.a.cus)
+    L.a.slots = L.a.cus;
   // One length for the whole batch and a segment count ((sequence, unit
   // block) pairs) that is a multiple of the persistent grid: the split gives
   // every group whole segments, so decode_main writes every row itself
