@@ -891,7 +891,7 @@ void decode_main(const DecodeArgs a) {
       // already in flight), unless the previous segment loaded them already.
       QRaw<D> qraw;
       int pg0;
-      constexpr bool kPartFirst = D > 64;   // (see below)
+      constexpr bool kPartFirst = D > 64 && !(D == 256 && QSplit<KV, QT>::value);   // (see below)
       int pgl = kPartFirst && nt > nfull ? page_id(nfull) : 0;
       if (kNext && x == seg_next) {
         qraw = q_next;
@@ -952,7 +952,8 @@ void decode_main(const DecodeArgs a) {
       // took 153 with one, so one group per CU: 256 log-normal lengths up to
       // 2000, 32/8 heads, 50.0 us against 43.8, 64 sequences of 500-2000
       // tokens, 16/16 heads, 51.1 against 43.5.  At one sequence of 1000 tokens
-      // it costs 0.6 us.)
+      // it costs 0.6 us.)  So does the split query at head_dim 256, which with it
+      // spilled 25 registers: 64 x 4096 tokens, 16/4 heads, 171.8 us against 164.9.
       auto load_part = [&](TileT& last) {
         load_tile<D, KV, ST, false, SV>(a, tile_ptr(t_first + nfull * P, pgl), lo,
                                            ntok - (t_first + nfull * P) * kTile, last, lane16, grp);

@@ -67,3 +67,9 @@ def pick(kernels, pattern):
 def test_head_dim_64_decode_fits_two_groups_per_cu(kernels, pattern):
     for name, k in pick(kernels, pattern).items():
         assert k[".vgpr_count"] <= 128, (name, k[".vgpr_count"])
+
+
+@pytest.mark.parametrize("kernel", ["decode_main"])
+def test_no_register_spills(kernels, kernel):
+    spills = {n: k[".vgpr_spill_count"] for n, k in pick(kernels, kernel + "I").items() if k[".vgpr_spill_count"]}
+    assert not spills
