@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
     float mb = M;
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
-      if (s0 + i >= a.nsplit) ms[i] = -INFINITY;         // (the last piece read again)
+      if (s0 + i >= a.nsplit) ms[i] = -INFINITY;         // (the last piece read again: left out below, as 0 x Inf is NaN)
       mb = fmaxf(mb, ms[i]);
     }
     const float mu = mb == -INFINITY ? 0.f : mb;         // (a piece without a key weighs 2^-inf = 0)
@@ -287,6 +287,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
     A *= r;
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
+      if (s0 + i >= a.nsplit) break;
       const float w = fast_exp2(ms[i] - mu);
       L += w * ls[i];
       A += w * x[i];

@@ -1112,7 +1112,7 @@ void decode_main(const DecodeArgs a) {
           float mb = M;
 #pragma unroll
           for (int p2 = 0; p2 < PB; ++p2) {
-            if (p0 + p2 > w1) mw[p2] = -INFINITY;           // (the last state read again)
+            if (p0 + p2 > w1) mw[p2] = -INFINITY;           // (the last state read again: left out below, as 0 x Inf is NaN)
             mb = fmaxf(mb, mw[p2]);
           }
           const float mref = mb == -INFINITY ? 0.f : mb;    // (a wave without a tile weighs 2^-inf = 0)
@@ -1121,6 +1121,7 @@ void decode_main(const DecodeArgs a) {
           A *= r;
 #pragma unroll
           for (int p2 = 0; p2 < PB; ++p2) {
+            if (p0 + p2 > w1) break;
             const float wt = fast_exp2(mw[p2] - mref);
             L += wt * lw[p2];
             A += wt * x[p2];

@@ -1195,14 +1195,14 @@ __global__ __launch_bounds__(256) void prefill_merge(const PrefillArgs a) {
     f32x4 x[kMergeBatch];
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      const int64_t r = min(s0 + k, a.nsplit - 1) * a.nrows + row;   // (past the last run: reread, weighed out)
+      const int64_t r = min(s0 + k, a.nsplit - 1) * a.nrows + row;   // (past the last run: reread)
       ml[k] = *(const float2*)(a.part_ml + 2 * r);
       x[k] = *(const f32x4*)(a.part_o + r * D + 4 * li);
     }
     float mb = M;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      if (s0 + k >= a.nsplit) ml[k].x = -INFINITY;
+      if (s0 + k >= a.nsplit) ml[k].x = -INFINITY;    // (left out below, as 0 x Inf is NaN)
       mb = fmaxf(mb, ml[k].x);
     }
     const float mref = mb == -INFINITY ? 0.f : mb;    // (no key seen yet: every weight is 2^-inf = 0)
@@ -1211,6 +1211,7 @@ __global__ __launch_bounds__(256) void prefill_merge(const PrefillArgs a) {
     A *= r0;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
+      if (s0 + k >= a.nsplit) break;
       const float w = fast_exp2(ml[k].x - mref);
       L += w * ml[k].y;
       A += w * x[k];
