@@ -1130,13 +1130,13 @@ void decode_main(const DecodeArgs a) {
         }
         const int hqo = hkv * a.G + 16 * hg + cc;
         if (direct) {
-          const float inv = 1.0f / (L == 0.f ? 1.f : L);
+          const float ls = L == 0.f ? 1.f : L;            // (A / L, not A times 1 / L: one rounding before the 16-bit one)
           char* op = a.out + b * a.o_sb + (int64_t)hqo * a.o_sh + DL * lane * (int)sizeof(uint16_t);
           if constexpr (DL == 1) {
-            store_out(QT{}, op, A[0] * inv);
+            store_out(QT{}, op, A[0] / ls);
           } else {
 #pragma unroll
-            for (int e = 0; e < DL; e += 2) *(uint32_t*)(op + 2 * e) = pack2(QT{}, A[e] * inv, A[e + 1] * inv);
+            for (int e = 0; e < DL; e += 2) *(uint32_t*)(op + 2 * e) = pack2(QT{}, A[e] / ls, A[e + 1] / ls);
           }
         } else {
           const int64_t ps = ((int64_t)pslot_id * NW + uin) * a.G16 + cc;
