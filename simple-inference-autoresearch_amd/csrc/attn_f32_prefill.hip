@@ -72,6 +72,7 @@ void attn_f32_prefill(const F32Args a) {
   const int lim = !live ? 0 : a.causal ? max(0, min(a.Tk, off + i)) : a.Tk;
   const int i_last = uniform(min(chunk * kF32TileCols + kF32TileCols - 1, a.ncol - 1) / a.G);
   const int hi = a.causal ? max(0, min(a.Tk, off + i_last)) : a.Tk;   // keys of the group's last column
+  const int lim0 = a.causal ? min(a.Tk, off + uniform(chunk * kF32TileCols / a.G)) : a.Tk;   // of its first one
 
   const char* qp = a.q + b * a.q_sb + (int64_t)(hkv * a.G + g) * a.q_sh + (int64_t)i * a.q_sm + 16 * h;
   // q operand: column l32, dims 8 j + 4 h + [0, 4) of piece j (dead columns
@@ -98,27 +99,25 @@ void attn_f32_prefill(const F32Args a) {
     for (int j = 0; j < n; ++j) k[j] = *(const f32x4*)(kp + 32 * (j0 + j));
   };
   // V operand of tile t: for S^T register j, key 8 (j / 4) + 4 h + j % 4 of
-  // the tile, the ET dimensions of row l32; registers [j0, j0 + n)
+  // the tile, EP of the ET dimensions of row l32; registers [j0, j0 + n), dimensions from e0 on
   // (past the last key: that row of the tile again, with zero weights)
-  auto load_v = [&](int t, float (*v)[ET], int j0, int n) {
-#pragma unroll
-    for (int j = 0; j < n; ++j) {
-      const int key = t * 32 + 8 * ((j0 + j) >> 2) + 4 * h + ((j0 + j) & 3);
-      const char* vp = vb + (int64_t)min(key, hi - 1) * a.v_sn + 4 * f32_dim<D>(D < 32 ? l32 & (D - 1) : l32, 0);
-      if constexpr (ET == 1) {
-        v[j][0] = *(const float*)vp;
-      } else if constexpr (ET == 2) {
-        const f32x2 x = *(const f32x2*)vp;
-        v[j][0] = x[0]; v[j][1] = x[1];
-      } else {
-#pragma unroll
-        for (int p = 0; p < ET / 4; ++p) {
-          const f32x4 x = *(const f32x4*)(vp + 512 * p);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[j][4 * p + e] = x[e];
-        }
-      }
+  constexpr int EP = ET < 4 ? ET : 4;            // 32-dimension tiles per V load
+  auto load_v1 = [&](int key, float* x, int e0) {
+    const char* vp = vb + (int64_t)key * a.v_sn + 4 * f32_dim<D>(D < 32 ? l32 & (D - 1) : l32, e0);
+    if constexpr (EP == 1) {
+      x[0] = *(const float*)vp;
+    } else if constexpr (EP == 2) {
+      const f32x2 y = *(const f32x2*)vp;
+      x[0] = y[0]; x[1] = y[1];
+    } else {
+      const f32x4 y = *(const f32x4*)vp;
+      x[0] = y[0]; x[1] = y[1]; x[2] = y[2]; x[3] = y[3];
     }
+  };
+  auto load_v = [&](int t, float (*v)[EP], int j0, int n, int e0) {
+#pragma unroll
+    for (int j = 0; j < n; ++j)
+      load_v1(min(t * 32 + 8 * ((j0 + j) >> 2) + 4 * h + ((j0 + j) & 3), hi - 1), v[j], e0);
   };
 
   f32x16 o[ET];
@@ -170,28 +169,61 @@ void attn_f32_prefill(const F32Args a) {
     }
     return part[0];
   };
-  // O^T over registers [j0, j0 + n) of the weights: 8 keys (4 MFMAs) from zero, then added
-  auto pv = [&](const float (*v)[ET], int j0, int n, const f32x16& s) {
+  // O^T over registers [j0, j0 + n) of the weights, one key at a time, each
+  // column taking only the keys that it sees
+  auto pv_each = [&](int t, int j0, int n, int e0, const f32x16& s) {
+    for (int q = 0; q < 2 * n; ++q) {
+      const int jr = j0 + (q >> 1), key = t * 32 + 8 * (jr >> 2) + 4 * (q & 1) + (jr & 3);
+      if (key >= hi) continue;
+      float p = 0.f, x[EP], lo, up;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) p = j == jr ? s[j] : p;
+      halves(p, lo, up);
+      p = q & 1 ? up : lo;
+      load_v1(key, x, e0);
+#pragma unroll
+      for (int e = 0; e < EP; ++e) {
+        const f32x16 part = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? x[e] : 0.f, h == 0 ? p : 0.f, f32x16{}, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[e0 + e][j] += key < lim ? part[j] : 0.f;
+      }
+    }
+  };
+  // The same: 8 keys (4 MFMAs) from zero, then added.  In a tile with keys that
+  // not every column sees (they weigh 0), values that are not finite go one
+  // key at a time, as 0 times those is NaN: so a hidden key's never reach a
+  // column, whichever columns share the group.
+  auto pv = [&](const float (*v)[EP], int t, int j0, int n, int e0, const f32x16& s) {
+    if (t * 32 + 31 >= lim0) {
+      uint32_t big = 0;
+#pragma unroll
+      for (int j = 0; j < n; ++j)
+#pragma unroll
+        for (int e = 0; e < EP; ++e) big = max(big, __builtin_bit_cast(uint32_t, v[j][e]) & 0x7fffffffu);
+      if (__any(big >= 0x7f800000u)) {
+        pv_each(t, j0, n, e0, s);
+        return;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < n; j += 4)
 #pragma unroll
-      for (int e = 0; e < ET; ++e) {
+      for (int e = 0; e < EP; ++e) {
         f32x16 part = f32x16{};
 #pragma unroll
         for (int i2 = 0; i2 < 4; ++i2)
           part = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j + i2][e], s[j0 + j + i2], part, 0, 0, 0);
-        o[e] += part;
-
+        o[e0 + e] += part;
       }
   };
   if constexpr (kAhead) {
     auto tile = [&](int t, const f32x4* k, f32x4* knext) {
-      float v[16][ET];
-      load_v(t, v, 0, 16);
+      float v[16][EP];
+      load_v(t, v, 0, 16, 0);
       if ((t + 4) * 32 < hi) load_k(t + 4, knext, 0, KQ);
       f32x16 s = qk(k, 0, std::integral_constant<int, KQ>{});
       softmax(t, s);
-      pv(v, 0, 16, s);
+      pv(v, t, 0, 16, 0, s);
     };
     f32x4 ka[KQ], kn[KQ];
     int t = wave;
@@ -203,15 +235,16 @@ void attn_f32_prefill(const F32Args a) {
   } else {
     constexpr int NC = D <= 128 ? D / 32 : 4;      // K and V in NC parts
     constexpr int KC = KQ / NC, VC = 16 / NC;      // K pieces and V registers per part
+    constexpr int NH = ET / EP, NV = NC * NH;      // V parts: VC registers, EP tiles of dimensions
     f32x4 k[2][KC];
-    float v[2][VC][ET];
+    float v[2][VC][EP];
     if (wave * 32 < hi) load_k(wave, k[0], 0, KC);
     for (int t = wave; t * 32 < hi; t += 4) {
       f32x16 s;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         if (c < NC - 1) load_k(t, k[(c + 1) & 1], (c + 1) * KC, KC);
-        else load_v(t, v[0], 0, VC);
+        else load_v(t, v[0], 0, VC, 0);
         __builtin_amdgcn_sched_barrier(0);
         {
           const f32x16 part = qk(k[c & 1], c * KC, std::integral_constant<int, KC>{});
@@ -222,11 +255,11 @@ void attn_f32_prefill(const F32Args a) {
       }
       softmax(t, s);
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        if (c < NC - 1) load_v(t, v[(c + 1) & 1], VC * (c + 1), VC);
+      for (int c = 0; c < NV; ++c) {
+        if (c < NV - 1) load_v(t, v[(c + 1) & 1], VC * ((c + 1) / NH), VC, EP * ((c + 1) % NH));
         else load_k(t + 4, k[0], 0, KC);           // (past the last tile: the last key again, unused)
         __builtin_amdgcn_sched_barrier(0);
-        pv(v[c & 1], VC * c, VC, s);
+        pv(v[c & 1], t, VC * (c / NH), VC, EP * (c % NH), s);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
