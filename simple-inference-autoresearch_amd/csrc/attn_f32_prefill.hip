@@ -193,8 +193,8 @@ void attn_f32_prefill(const F32Args a) {
   // not every column sees (they weigh 0), values that are not finite go one
   // key at a time, as 0 times those is NaN: so a hidden key's never reach a
   // column, whichever columns share the group.
-  auto pv = [&](const float (*v)[EP], int t, int j0, int n, int e0, const f32x16& s) {
-    if (t * 32 + 31 >= lim0) {
+  auto pv = [&](const float (*v)[EP], int t, int j0, int n, int e0, const f32x16& s, auto check) {
+    if (decltype(check)::value && t * 32 + 31 >= lim0) {
       uint32_t big = 0;
 #pragma unroll
       for (int j = 0; j < n; ++j)
@@ -223,7 +223,7 @@ void attn_f32_prefill(const F32Args a) {
       if ((t + 4) * 32 < hi) load_k(t + 4, knext, 0, KQ);
       f32x16 s = qk(k, 0, std::integral_constant<int, KQ>{});
       softmax(t, s);
-      pv(v, t, 0, 16, 0, s);
+      pv(v, t, 0, 16, 0, s, std::true_type{});
     };
     f32x4 ka[KQ], kn[KQ];
     int t = wave;
@@ -239,7 +239,7 @@ void attn_f32_prefill(const F32Args a) {
     f32x4 k[2][KC];
     float v[2][VC][EP];
     if (wave * 32 < hi) load_k(wave, k[0], 0, KC);
-    for (int t = wave; t * 32 < hi; t += 4) {
+    auto tile = [&](int t, auto check) {
       f32x16 s;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -259,10 +259,13 @@ void attn_f32_prefill(const F32Args a) {
         if (c < NV - 1) load_v(t, v[(c + 1) & 1], VC * ((c + 1) / NH), VC, EP * ((c + 1) % NH));
         else load_k(t + 4, k[0], 0, KC);           // (past the last tile: the last key again, unused)
         __builtin_amdgcn_sched_barrier(0);
-        pv(v[c & 1], t, VC * (c / NH), VC, EP * (c % NH), s);
+        pv(v[c & 1], t, VC * (c / NH), VC, EP * (c % NH), s, check);
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
+    };
+    int t = wave;
+    for (; t * 32 + 31 < lim0; t += 4) tile(t, std::false_type{});   // (with the check 2-4% slower from 512 tokens on)
+    for (; t * 32 < hi; t += 4) tile(t, std::true_type{});
   }
 
   // merge the 4 waves: every state scaled to the common max, then added
@@ -301,10 +304,14 @@ void attn_f32_prefill(const F32Args a) {
   if (wave < 2) add(sm_o[wave]);
   if (wave == 1) put(sm_o[1]);
   __syncthreads();
-  if (wave != 0 || !live) return;
+  if (wave != 0 || chunk * kF32TileCols + l32 >= a.ncol) return;
   add(sm_o[1]);
   const float inv = L == 0.f ? 0.f : 1.0f / L;     // no visible key: zeros (the reference's l_safe guard)
-  char* op = a.out + b * a.o_sb + (int64_t)(hkv * a.G + g) * a.o_sh + (int64_t)i * a.o_sm;
+  int c2 = (int)threadIdx.x & 31;
+  asm volatile("" : "+v"(c2));                     // (computed again: held through the loop, they were spilled)
+  c2 += chunk * kF32TileCols;
+  const int i2 = c2 / a.G;
+  char* op = a.out + b * a.o_sb + (int64_t)(hkv * a.G + c2 - i2 * a.G) * a.o_sh + (int64_t)i2 * a.o_sm;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int r = 8 * (j >> 2) + 4 * h + (j & 3);

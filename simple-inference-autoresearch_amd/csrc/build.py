@@ -84,12 +84,13 @@ def link_ext(obj: str) -> str:
     return out
 
 
-# Extra flags per source: the decode kernels keep their MFMA accumulators in
-# VGPRs (no AGPR round trips around the online-softmax rescale).
+# Extra flags per source: the decode kernels and the fp32 prefill keep their
+# MFMA results in VGPRs (no AGPR round trips around the online-softmax rescale).
 EXTRA_FLAGS = {
     "decode_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "decode_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "decode_i8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attn_f32_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

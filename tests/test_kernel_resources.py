@@ -69,7 +69,7 @@ def test_head_dim_64_decode_fits_two_groups_per_cu(kernels, pattern):
         assert k[".vgpr_count"] <= 128, (name, k[".vgpr_count"])
 
 
-@pytest.mark.parametrize("kernel", ["decode_main"])
+@pytest.mark.parametrize("kernel", ["decode_main", "attn_f32_prefill"])
 def test_no_register_spills(kernels, kernel):
     spills = {n: k[".vgpr_spill_count"] for n, k in pick(kernels, kernel + "I").items() if k[".vgpr_spill_count"]}
     assert not spills
