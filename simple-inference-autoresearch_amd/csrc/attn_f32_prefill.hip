@@ -189,10 +189,12 @@ void attn_f32_prefill(const F32Args a) {
       }
     }
   };
-  // The same: 8 keys (4 MFMAs) from zero, then added.  In a tile with keys that
-  // not every column sees (they weigh 0), values that are not finite go one
-  // key at a time, as 0 times those is NaN: so a hidden key's never reach a
-  // column, whichever columns share the group.
+  // The same: 8 keys (4 MFMAs) from zero, two such sums (one from head_dim 128
+  // on) added to O together.  (One by one, the error of 37 rows over 1500 keys
+  // was 2.0-2.1e-7 of the result up to head_dim 64, now 1.9e-7.)  In a tile
+  // with keys that not every column sees (they weigh 0), values that are not
+  // finite go one key at a time, as 0 times those is NaN: so a hidden key's
+  // never reach a column, whichever columns share the group.
   auto pv = [&](const float (*v)[EP], int t, int j0, int n, int e0, const f32x16& s, auto check) {
     if (decltype(check)::value && t * 32 + 31 >= lim0) {
       uint32_t big = 0;
@@ -206,14 +208,14 @@ void attn_f32_prefill(const F32Args a) {
       }
     }
 #pragma unroll
-    for (int j = 0; j < n; j += 4)
+    for (int j = 0; j < n; j += 8)
 #pragma unroll
       for (int e = 0; e < EP; ++e) {
-        f32x16 part = f32x16{};
+        f32x16 part[2] = {f32x16{}, f32x16{}};
 #pragma unroll
-        for (int i2 = 0; i2 < 4; ++i2)
-          part = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j + i2][e], s[j0 + j + i2], part, 0, 0, 0);
-        o[e0 + e] += part;
+        for (int i2 = 0; i2 < min(8, n); ++i2)
+          part[i2 >> 2] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j + i2][e], s[j0 + j + i2], part[i2 >> 2], 0, 0, 0);
+        o[e0 + e] += n > 4 ? part[0] + part[1] : part[0];
       }
   };
   if constexpr (kAhead) {
