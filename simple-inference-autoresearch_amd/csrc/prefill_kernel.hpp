@@ -1104,6 +1104,7 @@ void prefill_fwd(const PrefillArgs a) {
       issue_k(0, lk0);
       char* qst = ((wave >> 1) == 0 ? lv0 : lv1) + (wave & 1) * 32 * RB;
       dma_q(qst);
+      __builtin_amdgcn_sched_barrier(0);                  // (the wait counts K_1's transfers as the newest)
       issue_k(1, lk1);
       wait_vmcnt<NK>();                                   // this wave's K_0 and q landed
       read_q(qst);
