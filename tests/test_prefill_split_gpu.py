@@ -106,6 +106,14 @@ def test_split_equals_whole_and_oracle(gpu_pkg, D, dtype, shape, causal, layout)
     assert torch.equal(tm.transpose(1, 2), out)
 
 
+def assert_eight_wave_runs(lm, q, k, runs):
+    """These tensors are cut into `runs` runs on variant 4, which needs the V^T images as well as the partials (variant
+    3, the 4-wave groups that convert V in LDS, needs the partials alone)."""
+    B, Hq, Tq, D = q.shape
+    n_whole, n_split = workspace_sizes(lm, q, k)
+    assert n_split == n_whole + B * Hq * Tq * runs * (D + 2) * 4, (n_whole, n_split)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("Tq,Tk", [(512, 8192), (500, 6001)])
 def test_split_eight_wave_groups(gpu_pkg, Tq, Tk):
@@ -113,6 +121,7 @@ def test_split_eight_wave_groups(gpu_pkg, Tq, Tk):
     lm = import_module("simple-inference-autoresearch_amd._lib")
     announce(f"prefill split 8 waves {Tq} {Tk}")
     q, k, v = inputs(1, 32, 8, Tq, Tk, 128, torch.bfloat16, "plain", seed=Tk)
+    assert_eight_wave_runs(lm, q, k, 4)
     out = gpu_pkg.attention_flash_triton(q, k, v, causal=True)
     check_all(out, whole_call(lm, q, k, v, True), q, k, v, True, f"8 waves {Tq} {Tk}")
 
@@ -134,6 +143,27 @@ def test_split_rotary_prologue(gpu_pkg, D, dtype, interleaved, table):
     qr, _ = gpu_pkg.rope_triton(q.transpose(1, 2), q.transpose(1, 2), cos[start:], sin[start:],
                                 interleaved=interleaved)
     assert torch.equal(out, gpu_pkg.attention_flash_triton(qr.transpose(1, 2), k, v, causal=True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("table", ["same", "fp32"])
+def test_split_eight_wave_rotary_prologue(gpu_pkg, interleaved, table):
+    """The same at the prompt chunks and prefixes that run the 8-wave groups (bf16, head_dim 128)."""
+    lm = import_module("simple-inference-autoresearch_amd._lib")
+    announce(f"prefill split rope 8 waves interleaved={interleaved} {table}")
+    T, start, D = 500, 6001, 128
+    q, k, v = inputs(1, 32, 8, T, start + T, D, torch.bfloat16, "token_major", seed=start)
+    assert_eight_wave_runs(lm, q, k, 4)
+    rf = gpu_pkg.RopeFrequencies(D, start + T, device=torch.device(DEV))
+    cos, sin = rf.get(start + T, dtype=torch.bfloat16 if table == "same" else torch.float32)
+    out = gpu_pkg.rope_attention_flash_triton(q, k, v, cos, sin, causal=True, start_offset=start,
+                                              interleaved=interleaved)
+    qr, _ = gpu_pkg.rope_triton(q.transpose(1, 2), q.transpose(1, 2), cos[start:], sin[start:],
+                                interleaved=interleaved)
+    qr = qr.transpose(1, 2)
+    check_all(out, whole_call(lm, qr, k, v, True), qr, k, v, True, f"8 waves rope {table}")
+    assert torch.equal(out, gpu_pkg.attention_flash_triton(qr, k, v, causal=True))
 
 
 @pytest.mark.gpu
