@@ -38,6 +38,7 @@
 #pragma once
 
 #include "sia_common.hpp"
+#include "sk_split.hpp"
 
 namespace sia {
 
@@ -215,41 +216,9 @@ __device__ int plan_work(const DecodeArgs& a, int* pre, int* red, int tok0, int&
   return uniform(pre[a.B]);
 }
 
-// Stream-K split of W tiles over G work-groups: group g takes
-// [lo(g), lo(g+1)) with lo(g) = floor(g W / G).  With W = Q G + R this is
-// g Q + floor(g R / G), and g R < G^2 (G is at most the persistent grid, some
-// thousand) stays below 2^24, where one fp32 product and a correction divide
-// exactly.  (The 64-bit divisions this replaces took ~0.4 us of every group's
-// start at one sequence of 1000 tokens.)
-struct SkSplit {
-  int W, G, Q, R;
-  float rG;            // 1 / G
-};
+// The split of the work line (see sk_split.hpp), with v_rcp_f32's reciprocals.
 __device__ __forceinline__ SkSplit sk_split(int W, int G) {
-  SkSplit s;
-  s.W = W;
-  s.G = G;
-  s.Q = (int)((uint32_t)W / (uint32_t)G);
-  s.R = W - s.Q * G;
-  s.rG = __builtin_amdgcn_rcpf((float)G);
-  return s;
-}
-__device__ __forceinline__ int sk_lo(const SkSplit& s, int g) {
-  const int n = g * s.R;
-  int q = (int)((float)n * s.rG);
-  const int r = n - q * s.G;
-  q += r >= s.G ? 1 : r < 0 ? -1 : 0;
-  return g * s.Q + q;
-}
-// The group holding position x (0 <= x < W), the last one with lo(g) <= x:
-// ceil((x + 1) G / W) - 1 by an fp32 estimate, within one of it (the error is
-// below G 2^-21), set right by the bounds.
-__device__ __forceinline__ int sk_group(const SkSplit& s, int x) {
-  int g = (int)ceilf((float)(x + 1) * ((float)s.G * __builtin_amdgcn_rcpf((float)s.W))) - 1;
-  g = min(max(g, 0), s.G - 1);
-  if (g > 0 && sk_lo(s, g) > x) --g;
-  if (g + 1 < s.G && sk_lo(s, g + 1) <= x) ++g;
-  return g;
+  return sk_split(W, G, __builtin_amdgcn_rcpf((float)G), __builtin_amdgcn_rcpf((float)W));
 }
 
 // -------------------------------------------------------------- tile data

@@ -63,7 +63,7 @@ int launch_decode_typed(DecodeLaunch& L) {
   if (occ <= 0) return fail(SIA_ERR_LAUNCH, "decode kernel does not fit on a CU (LDS %zu B)", lds);
   L.a.cus = device_info().cus;
   L.a.slots = L.a.cus * occ;
-  if (L.a.slots > 4095) L.a.slots = 4095;   // (the split's 24-bit arithmetic, sk_lo)
+  if (L.a.slots > kMaxSplitGroups) L.a.slots = kMaxSplitGroups;
   // int8 K/V at one shared length: one group per CU, also where two fit
   // (head_dim 64).  No ragged starts for the second to hide (see
   // kTwoGroupTiles), and a grid twice as large costs: fp16 scales, 32/8 heads,
