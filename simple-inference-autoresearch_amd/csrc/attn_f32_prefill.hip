@@ -197,12 +197,13 @@ void attn_f32_prefill(const F32Args a) {
   // never reach a column, whichever columns share the group.
   auto pv = [&](const float (*v)[EP], int t, int j0, int n, int e0, const f32x16& s, auto check) {
     if (decltype(check)::value && t * 32 + 31 >= lim0) {
-      uint32_t big = 0;
+      float z[4] = {0.f, 0.f, 0.f, 0.f};               // (0 x Inf and 0 x NaN are NaN, and stay)
 #pragma unroll
       for (int j = 0; j < n; ++j)
 #pragma unroll
-        for (int e = 0; e < EP; ++e) big = max(big, __builtin_bit_cast(uint32_t, v[j][e]) & 0x7fffffffu);
-      if (__any(big >= 0x7f800000u)) {
+        for (int e = 0; e < EP; ++e) z[(j * EP + e) & 3] = __builtin_fmaf(v[j][e], 0.f, z[(j * EP + e) & 3]);
+      const float any = (z[0] + z[1]) + (z[2] + z[3]);
+      if (__any(any != any)) {
         pv_each(t, j0, n, e0, s);
         return;
       }
