@@ -4,7 +4,7 @@
 // products in fp32 end to end.  On the vector ALUs every key row cost a
 // column D/4 lanes' products plus log2(D/4) cross-lane sums: one sequence of
 // 512 tokens, 32/8 heads, head_dim 64 (1.08 GFLOP) took 113.8 us at 9.5
-// TFLOP/s; here 18.7 us.
+// TFLOP/s; here 19.1 us.
 //
 // A work-group covers 32 columns, (query row, query head) pairs of one KV
 // head in row-major order, so a causal group of G = 4 spans 8 rows.  Its 4

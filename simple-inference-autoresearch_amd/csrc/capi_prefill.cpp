@@ -60,6 +60,8 @@ struct KeySplit {
 // 512 + 8192 136 -> 84; head_dim 256 200 + 6000 176 -> 48; prompts without a
 // prefix stay whole (512 tokens 15.5 against 25 us in two runs, 1024 25
 // against 39: the partials and the merge cost more than the chain saves).
+// Two groups per CU are counted at head_dim 64, where the registers hold
+// three: the constants were fitted so.
 KeySplit key_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t Tk, int64_t D, bool bf16, int cus) {
   KeySplit best;
   const int64_t nkb = (Tk + kPfBN - 1) / kPfBN;

@@ -116,10 +116,11 @@ constexpr int kBufferFlags = 0x00020000;   // gfx9 raw buffer resource word 3 (3
 //    merge the runs' fp32 partials in prefill_merge: few query rows over many
 //    keys, where whole calls leave most CUs idle (chosen by key_splits in
 //    capi_prefill.cpp, which holds the measurements).
-//  * D <= 64: 4 waves with the same register budget, so two work-groups share
-//    a CU and one's prologue and epilogue overlap the other's key loop (MHA
-//    D = 64 at T = 1024: 88 -> 70 us per call); a two-stage ring at D = 64,
-//    four stages below, where blocks are small (measured best of the two).
+//  * D <= 64: 4 waves with the same register budget (137-165 are used), so
+//    three work-groups share a CU and one's prologue and epilogue overlap the
+//    others' key loops (MHA D = 64 at T = 1024: 88 -> 70 us per call when it
+//    was two); a two-stage ring at D = 64, four stages below, where blocks are
+//    small (measured best of the two).
 //  * D = 256: the O^T accumulators alone take 128 registers per lane, so 4
 //    waves run one per SIMD with 512 registers, and the 32 KB blocks fit LDS
 //    as a two-stage ring.
@@ -596,14 +597,6 @@ void prefill_fwd(const PrefillArgs a) {
 #pragma unroll
   for (int j = 0; j < KST; ++j) k_rd[j] = l32 * RB + (((2 * j + h) ^ (l32 % NC)) * 16);
 
-  // DMA of K block `blk` / V^T image `blk` into its ring stage (blk % S):
-  // wave w moves 1 KB pieces [w NK, (w+1) NK) of the block (rows past Tk
-  // read as zero through the buffer bound) and the same range of the image.
-  // A block past the work-group's last one, and a piece past the block's end
-  // (waves beyond the DMA count at small head_dim), is issued with an empty
-  // buffer range: the hardware drops every out-of-range read (no memory
-  // traffic) and what it fills is never read, so every wave issues the same
-  // instruction count per group and the waits below are constants.
   // kQLds: q comes through LDS, a wave's 32 rows by 1 KB LDS DMA (whole rows,
   // swizzled like the K stages) into a part of the ring that the first blocks
   // do not use yet, then read in the operand layout.  Loaded straight into
@@ -630,8 +623,16 @@ void prefill_fwd(const PrefillArgs a) {
 #pragma unroll
     for (int j = 0; j < KST; ++j) qop[j] = *(const u32x4*)(qst + k_rd[j]);
   };
-  // (one transfer instruction each: the ring refills are spread over the
-  // MFMA stream, see `qk`)
+  // DMA of K block `blk` / V^T image `blk` into its ring stage (blk % S):
+  // wave w moves 1 KB pieces [w NK, (w+1) NK) of the block (rows past Tk
+  // read as zero through the buffer bound) and the same range of the image.
+  // A block past the work-group's last one, and a piece past the block's end
+  // (waves beyond the DMA count at small head_dim), is issued with an empty
+  // buffer range: the hardware drops every out-of-range read (no memory
+  // traffic) and what it fills is never read, so every wave issues the same
+  // instruction count per group and the waits below are constants.
+  // (issue_k1 and issue_v1: one transfer instruction each, as the ring refills
+  // are spread over the MFMA stream, see `qk`)
   auto issue_k1 = [&](int blk, char* LK, int i) {
     const bool live = blk < nblk;
     const int key0 = live ? blk * kPfBN : 0;
