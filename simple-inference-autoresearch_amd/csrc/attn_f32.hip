@@ -277,11 +277,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
     float mb = M;
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
-      if (s0 + i >= a.nsplit) {                          // (the last piece read again: left out, as 0 x Inf is NaN)
-        ms[i] = -INFINITY;
-        ls[i] = 0.f;
-        x[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      if (s0 + i >= a.nsplit) ms[i] = -INFINITY;         // (the last piece read again)
       mb = fmaxf(mb, ms[i]);
     }
     const float mu = mb == -INFINITY ? 0.f : mb;         // (a piece without a key weighs 2^-inf = 0)
@@ -292,7 +288,8 @@ __global__ __launch_bounds__(256) void attn_f32_merge(const F32Args a) {
     for (int i = 0; i < PB; ++i) {
       const float w = fast_exp2(ms[i] - mu);
       ls[i] *= w;
-      x[i] *= w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[i][e] = w * keep_below(x[i][e], s0 + i, a.nsplit);
     }
 #pragma unroll
     for (int o = 1; o < PB; o *= 2)

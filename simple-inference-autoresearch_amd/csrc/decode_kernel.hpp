@@ -1081,7 +1081,7 @@ void decode_main(const DecodeArgs a) {
           float mb = M;
 #pragma unroll
           for (int p2 = 0; p2 < PB; ++p2) {
-            if (p0 + p2 > w1) mw[p2] = -INFINITY;           // (the last state read again: left out below, as 0 x Inf is NaN)
+            if (p0 + p2 > w1) mw[p2] = -INFINITY;           // (the last state read again)
             mb = fmaxf(mb, mw[p2]);
           }
           const float mref = mb == -INFINITY ? 0.f : mb;    // (a wave without a tile weighs 2^-inf = 0)
@@ -1090,10 +1090,10 @@ void decode_main(const DecodeArgs a) {
           A *= r;
 #pragma unroll
           for (int p2 = 0; p2 < PB; ++p2) {
-            if (p0 + p2 > w1) break;
             const float wt = fast_exp2(mw[p2] - mref);
             L += wt * lw[p2];
-            A += wt * x[p2];
+#pragma unroll
+            for (int e = 0; e < DL; ++e) A[e] += wt * keep_below(x[p2][e], p0 + p2, w1 + 1);
           }
           M = mb;
         }

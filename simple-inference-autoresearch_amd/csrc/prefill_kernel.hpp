@@ -1204,7 +1204,7 @@ __global__ __launch_bounds__(256) void prefill_merge(const PrefillArgs a) {
     float mb = M;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      if (s0 + k >= a.nsplit) ml[k].x = -INFINITY;    // (left out below, as 0 x Inf is NaN)
+      if (s0 + k >= a.nsplit) ml[k].x = -INFINITY;
       mb = fmaxf(mb, ml[k].x);
     }
     const float mref = mb == -INFINITY ? 0.f : mb;    // (no key seen yet: every weight is 2^-inf = 0)
@@ -1213,10 +1213,10 @@ __global__ __launch_bounds__(256) void prefill_merge(const PrefillArgs a) {
     A *= r0;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      if (s0 + k >= a.nsplit) break;
       const float w = fast_exp2(ml[k].x - mref);
       L += w * ml[k].y;
-      A += w * x[k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A[e] += w * keep_below(x[k][e], s0 + k, a.nsplit);
     }
     M = mb;
   }

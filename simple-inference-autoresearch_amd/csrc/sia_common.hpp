@@ -140,6 +140,13 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // x / d = (umulhi(x, m) + x) >> l for 0 <= x < 2^32; the sum fits 32 bits
 // because callers keep x < 2^31.  The scalar unit does it in three
 // instructions instead of the ~25 dependent ones of a runtime division.
+// x where i < n, else 0: for a batch's copies past its last piece, whose weight
+// 0 does not rid them of an Inf.  By a mask, not by a condition: around a
+// condition the compiler moves the loads into branches, one round trip each.
+__device__ __forceinline__ float keep_below(float x, int i, int n) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, x) & ((i - n) >> 31));
+}
+
 struct FastDiv {
   uint32_t m;
   uint32_t l;
