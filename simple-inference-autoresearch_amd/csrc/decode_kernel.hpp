@@ -83,7 +83,6 @@ struct DecodeArgs {
   int32_t tps_force;
   int32_t seg_pen;                                   // virtual tiles charged to each segment start (the split)
   int32_t slots;                                     // persistent work-groups of decode_main
-  int32_t cus;                                       // CUs
   int32_t scale_vec;                                 // scale rows allow one vector load per lane
   int32_t direct_only;                               // no decode_reduce follows: empty calls write zeros here
   // 32-bit copies of the per-tile strides (bytes): page strides (0 when
@@ -91,6 +90,7 @@ struct DecodeArgs {
   // products
   uint32_t k_pg, v_pg, ks_pg, vs_pg;
   uint32_t k_tok, v_tok, ks_tok, vs_tok;
+  int32_t cus;                                       // CUs
 };
 
 // --------------------------------------------------------------------- plan
@@ -709,9 +709,10 @@ void decode_main(const DecodeArgs a) {
   G = min(G, max(1, a.max_items / 2));                      // two partial slots per group
   // (one segment per CU, all of one length: whole segments, nothing to merge,
   // 20.3 against 22.9 us at 64 x 1024 tokens)
-  if (std::is_same<KV, I8>::value && a.tps_force <= 0 && G > a.cus &&
-      (W < kTwoGroupTiles * shape.P * G || (pen == 0 && a.B * a.UB == a.cus)))
-    G = min(G, max(a.cus, a.B * a.UB));
+  if constexpr (D == 64 && std::is_same<KV, I8>::value)
+    if (a.tps_force <= 0 && G > a.cus &&
+        (W < kTwoGroupTiles * shape.P * G || (pen == 0 && a.B * a.UB == a.cus)))
+      G = min(G, max(a.cus, a.B * a.UB));
   const int nt0 = (tok0 + kTile - 1) / kTile;               // (one shared length)
   if (!a.kv_per_seq && a.tps_force <= 0) G = aligned_groups(a, nt0, G, shape.P, KV::bytes * D);
   if (blockIdx.x == 0) {

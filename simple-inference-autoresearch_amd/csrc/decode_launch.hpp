@@ -68,7 +68,7 @@ int launch_decode_typed(DecodeLaunch& L) {
   // (head_dim 64).  No ragged starts for the second to hide (see
   // kTwoGroupTiles), and a grid twice as large costs: fp16 scales, 32/8 heads,
   // 32 x 512 tokens 9.7 against 11.6 us, 256 x 1000 56.5 against 58.8.
-  if (std::is_same<KV, I8>::value && !L.a.kv_per_seq && L.a.tps_force == 0 && L.a.slots > L.a.cus)
+  if (D == 64 && std::is_same<KV, I8>::value && !L.a.kv_per_seq && L.a.tps_force == 0 && L.a.slots > L.a.cus)
     L.a.slots = L.a.cus;
   // One length for the whole batch and a segment count ((sequence, unit
   // block) pairs) that is a multiple of the persistent grid: the split gives
